@@ -43,11 +43,15 @@ __host__ __device__ inline int64_t o_at(const GdrArgs &a, int64_t tok, int64_t h
 bool gdr_strides_ok(const dm_gdr_desc *d, bool step);
 bool gdr_strides_16b(const dm_gdr_desc *d);
 
-// The generic kernels' workspace: the plan, then per (chunk, head) f32 intermediates.
+// The f32 kernels' workspace: the plan, then per (chunk, head) f32 intermediates, rows of KP and
+// VP columns (Dk and Dv padded with zeros to multiples of 64); names ending in T are transposed.
 struct GdrWs {
-    int32_t *seq_chunk0, *chunk_seq, *chunk_tok0, *chunk_len;
-    float *G, *qn, *kn, *W, *U, *Sc, *Vn;
-    float *Tm, *Am, *dvl, *dSn, *dVn, *ds, *gq, *gk, *gx;
+    int64_t KP, VP, npart;
+    int32_t *seq_chunk0, *chunk_seq, *chunk_tok0, *chunk_len, *seq_order;
+    double *G;  // cumulative log-decay
+    float *qn, *kn, *vp, *P, *W, *KT, *UT, *ScT, *VnT;
+    // the backward's
+    float *inv, *dop, *Tm, *Am, *WT, *dvlT, *F, *dSnT, *dVnT, *DPd, *dae, *gq, *gk, *dw, *dgv, *part;
 };
 
 int check_gdr(const dm_gdr_desc *d, const char *op, bool step);

@@ -60,6 +60,12 @@ __device__ __forceinline__ f32x4_t mfma16(const Frag8 &a, const Frag8 &b, const 
     }
 }
 
+// v_mfma_f32_16x16x4_f32: D[16x16] += A[16x4] B[4x16] in f32; lane l holds A's row (l % 16) and
+// B's column (l % 16) at k = l / 16; D as the 16x16x32 products'.
+__device__ __forceinline__ f32x4_t mfma4(float a, float b, const f32x4_t &c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
 // f32 -> 16-bit bits, two at a time: v_cvt_pk_bf16_f32 (round to nearest even) or
 // v_cvt_pk_f16_f32.
 typedef float f32x2_t __attribute__((ext_vector_type(2)));

@@ -12,9 +12,13 @@ void fill_f32(float *p, float value, int64_t n, hipStream_t st);
 void fill_zero(void *p, size_t bytes, hipStream_t st);
 
 int check_attention(const dm_attention_desc *d, const char *op);
-int launch_attn_fwd_generic(const MaskInfo &m, const dm_attention_desc *d, float scale,
-                            const void *q, const void *k, const void *v, void *o, float *lse,
-                            hipStream_t st);
+// f32 arithmetic, any dtype and head width up to 256 (attention_f32.hip).
+int launch_attn_fwd_f32(const MaskInfo &m, const dm_attention_desc *d, float scale, const void *q,
+                        const void *k, const void *v, void *o, float *lse, hipStream_t st);
+size_t attn_bwd_f32_workspace(const dm_attention_desc *d);
+int launch_attn_bwd_f32(const MaskInfo &m, const dm_attention_desc *d, float scale, const void *q,
+                        const void *k, const void *v, const void *o, const float *lse, const void *d_o,
+                        void *dq, void *dk, void *dv, void *workspace, hipStream_t st);
 
 // MFMA paths (attention_fwd.hip, attention_mfma_bwd.hip): bf16/f16, D in {64, 128}.
 bool rows_fit_32bit(const Strd &x, int64_t rows, int64_t d);

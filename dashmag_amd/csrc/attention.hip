@@ -51,15 +51,12 @@ using namespace dm;
 extern "C" {
 
 size_t dm_attention_fwd_workspace(const dm_attention_desc *desc) {
-    (void)desc;
-    return 0;
+    return desc ? mfma_fwd_workspace(desc) : 0;
 }
 
 int dm_attention_fwd(const dm_attention_desc *desc, const void *q, const void *k, const void *v,
                      void *o, float *lse, void *workspace, size_t workspace_bytes,
                      void *stream) {
-    (void)workspace;
-    (void)workspace_bytes;
     int rc = check_attention(desc, "attention");
     if (rc) return rc;
     hipStream_t st = (hipStream_t)stream;
@@ -75,7 +72,7 @@ int dm_attention_fwd(const dm_attention_desc *desc, const void *q, const void *k
         return DM_OK;
     }
     if (mfma_fwd_takes(desc, q, k, v))
-        return launch_attn_fwd_mfma(m, desc, scale, q, k, v, o, lse, st);
+        return launch_attn_fwd_mfma(m, desc, scale, q, k, v, o, lse, workspace, workspace_bytes, st);
     return launch_attn_fwd_f32(m, desc, scale, q, k, v, o, lse, st);
 }
 

@@ -16,7 +16,9 @@
 // staged into the other LDS slots during step j, from registers loaded one step earlier.
 // A wavefront skips the products and softmax of a tile none of its queries sees (it still takes
 // part in every barrier); the per-element mask runs only on tiles its rows' intervals cut.
+#include <algorithm>
 #include <string>
+#include <utility>
 
 #include "attention_kernels.h"
 #include "mfma.h"
@@ -28,6 +30,11 @@ namespace dm {
 // registers, more than two wavefronts per SIMD hold)
 template <int D>
 constexpr int fwd_waves() { return D == 256 ? 4 : 8; }
+// Wavefronts a SIMD the registers are held to. At width 64 128 registers (of 140 taken freely)
+// let two workgroups share a compute unit: unmasked 6144 queries and keys of 32 heads 420 -> 365 us,
+// of 128 heads 1470 -> 1264 us (841 -> 979 TFLOP/s).
+template <int D>
+constexpr int fwd_simd_waves() { return D == 64 ? 4 : 1; }
 constexpr int kFwdN = 64;   // keys per tile
 
 // Row strides (elements) of the LDS tiles: K rows are read along D by ds_read_b128 (16 lanes on
@@ -65,14 +72,39 @@ __device__ uint64_t dm_trace_fwd[2][256][4];
     } while (0)
 #endif
 
-template <int DT, int D, bool PAD>
-__global__ __launch_bounds__(64 * fwd_waves<D>(), 1) void attn_fwd_mfma(MaskInfo m, int64_t B, int64_t Hq,
+// A call whose work items leave compute units idle is split along the keys: the key tiles of a query
+// tile are cut into segments, a workgroup each, whose unnormalised outputs and (reference, sum)
+// pairs attn_fwd_merge combines; a query tile of one segment writes its outputs itself. The query
+// tiles are counted from the longest (last) down; tile t has the segments first[t] .. first[t + 1] - 1,
+// and workgroup x runs segment x / rows of the (batch row, head) x % rows.
+constexpr int kSplitTiles = 256;  // most query tiles of a split call
+struct FwdSplit {
+    int32_t nseg;  // segments of a (batch row, head); 0: the call is not split
+    float *o;      // [nseg][rows][queries of a tile][D]
+    float2 *ml;    // [nseg][rows][queries of a tile]
+    uint16_t first[kSplitTiles + 1];
+};
+// the query tile (from the longest down) of segment c
+__device__ __forceinline__ int split_tile(const FwdSplit &sp, int ntiles, int c) {
+    int lo = 0, hi = ntiles - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (sp.first[mid] <= c)
+            lo = mid;
+        else
+            hi = mid - 1;
+    }
+    return lo;
+}
+
+template <int DT, int D, bool PAD, bool SPLIT>
+__global__ __launch_bounds__(64 * fwd_waves<D>(), fwd_simd_waves<D>()) void attn_fwd_mfma(MaskInfo m, int64_t B, int64_t Hq,
                                                       int64_t Hkv, float scale, AttnStrides sd,
                                                       const uint16_t *__restrict__ q,
                                                       const uint16_t *__restrict__ k,
                                                       const uint16_t *__restrict__ v,
                                                       uint16_t *__restrict__ o,
-                                                      float *__restrict__ lse) {
+                                                      float *__restrict__ lse, FwdSplit sp) {
     constexpr int KS = FwdStrides<D>::K, VS = FwdStrides<D>::V;
     __shared__ FwdSmem<D> sm;
     constexpr int KSTEPS = D / 16;  // k-steps of S^T over the head dimension
@@ -80,7 +112,7 @@ __global__ __launch_bounds__(64 * fwd_waves<D>(), 1) void attn_fwd_mfma(MaskInfo
     constexpr int NW = fwd_waves<D>(), NT = 64 * NW, kFwdM = 32 * NW;
     const int64_t Tq = m.tq, Tk = m.tk;
     const int64_t ntiles = (Tq + kFwdM - 1) / kFwdM;
-    const int64_t nwork = ntiles * Hq * B;
+    const int64_t nwork = SPLIT ? sp.nseg * Hq * B : ntiles * Hq * B;
     const int64_t work = blockIdx.x;
     if (work >= nwork) return;
     // the key-value head is the fastest index (consecutive workgroups go to consecutive XCDs: with
@@ -88,8 +120,16 @@ __global__ __launch_bounds__(64 * fwd_waves<D>(), 1) void attn_fwd_mfma(MaskInfo
     // then the query tiles from the longest (last) down, then the batch row
     const int64_t kh = work % Hkv;
     const int64_t h = kh * (Hq / Hkv) + (work / Hkv) % (Hq / Hkv);
-    const int64_t tile = ntiles - 1 - (work / Hq) % ntiles;
-    const int64_t b = work / (Hq * ntiles);
+    int64_t tile = ntiles - 1 - (work / Hq) % ntiles;
+    int64_t b = work / (Hq * ntiles);
+    int32_t seg = 0, nseg = 1;
+    if constexpr (SPLIT) {
+        const int c = (int)(work / (Hq * B)), t = split_tile(sp, (int)ntiles, c);
+        seg = c - sp.first[t];
+        nseg = sp.first[t + 1] - sp.first[t];
+        tile = ntiles - 1 - t;
+        b = (work / Hq) % B;
+    }
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const bool first = NW == 4 || wave < 4;  // products first in each step
@@ -133,7 +173,12 @@ __global__ __launch_bounds__(64 * fwd_waves<D>(), 1) void attn_fwd_mfma(MaskInfo
     const int32_t my_hi = __builtin_amdgcn_readfirstlane(sm.hi[wave]);
     const int32_t my_flo = __builtin_amdgcn_readfirstlane(sm.flo[wave]);
     const int32_t my_fhi = __builtin_amdgcn_readfirstlane(sm.fhi[wave]);
-    const int32_t nt = kv_lo < kv_hi ? (kv_hi - kv_lo + kFwdN - 1) / kFwdN : 0;
+    int32_t nt = kv_lo < kv_hi ? (kv_hi - kv_lo + kFwdN - 1) / kFwdN : 0;
+    if constexpr (SPLIT) {
+        const int32_t per = (nt + nseg - 1) / nseg, t0 = seg * per;
+        kv_lo += t0 * kFwdN;
+        nt = max(0, min(per, nt - t0));
+    }
 
     // this wavefront's queries as the B operand: col = query, k = head dimension
     Frag8 qf[KSTEPS];
@@ -330,6 +375,19 @@ __global__ __launch_bounds__(64 * fwd_waves<D>(), 1) void attn_fwd_mfma(MaskInfo
     // finish: l over both halves, normalise, write O and lse
     const float ltot = lrow + __shfl_xor(lrow, 32, 64);
     if (!qvalid) return;
+    if constexpr (SPLIT) {
+        if (nseg > 1) {
+            const int64_t row = work * kFwdM + wave * 32 + col;
+#pragma unroll
+            for (int dt = 0; dt < DT32; dt++)
+#pragma unroll
+                for (int g4 = 0; g4 < 4; g4++)
+                    *(float4 *)(sp.o + row * D + dt * 32 + g4 * 8 + half * 4) =
+                        make_float4(acc[dt][g4 * 4], acc[dt][g4 * 4 + 1], acc[dt][g4 * 4 + 2], acc[dt][g4 * 4 + 3]);
+            if (half == 0) sp.ml[row] = make_float2(mc, ltot);
+            return;
+        }
+    }
     const float inv = ltot > 0.f ? 1.f / ltot : 0.f;
     uint16_t *op = o + ((b * Tq + qi) * Hq + h) * D;
 #pragma unroll
@@ -345,6 +403,44 @@ __global__ __launch_bounds__(64 * fwd_waves<D>(), 1) void attn_fwd_mfma(MaskInfo
     if (half == 0)
         lse[(b * Tq + qi) * Hq + h] =
             ltot > 0.f ? (float)((double)mc * 0.6931471805599453 + log((double)ltot)) : -INFINITY;
+}
+
+// The segments of the query tiles that have more than one, combined: D / 4 lanes a row, a lane four
+// columns, the segments added in order.
+template <int DT, int D>
+__global__ __launch_bounds__(256) void attn_fwd_merge(int64_t Tq, int64_t Hq, int64_t Hkv, int64_t B,
+                                                      int ntiles, FwdSplit sp, uint16_t *__restrict__ o,
+                                                      float *__restrict__ lse) {
+    constexpr int kFwdM = 32 * fwd_waves<D>(), L = D / 4, R = 256 / L;
+    const int64_t rows = Hq * B, x = blockIdx.x % rows;
+    const int t = (int)(blockIdx.x / rows), c0 = sp.first[t], nseg = sp.first[t + 1] - c0;
+    if (nseg < 2) return;
+    // the head and batch row, as attn_fwd_mfma takes them
+    const int64_t h = (x % Hkv) * (Hq / Hkv) + (x / Hkv) % (Hq / Hkv), b = x / Hq;
+    const int r = blockIdx.y * R + threadIdx.x / L, c = 4 * (threadIdx.x % L);
+    const int64_t qi = (int64_t)(ntiles - 1 - t) * kFwdM + r;
+    if (qi >= Tq) return;
+    const int64_t row0 = (c0 * rows + x) * kFwdM + r, step = rows * kFwdM;
+    float mc = -INFINITY;
+    for (int s = 0; s < nseg; s++) mc = fmaxf(mc, sp.ml[row0 + s * step].x);
+    const float ref = mc == -INFINITY ? 0.f : mc;
+    float l = 0.f, y[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < nseg; s++) {
+        const float2 ml = sp.ml[row0 + s * step];
+        const float4 v = *(const float4 *)(sp.o + (row0 + s * step) * D + c);
+        const float f = fast_exp2(ml.x - ref);
+        l += ml.y * f;
+        y[0] += v.x * f;
+        y[1] += v.y * f;
+        y[2] += v.z * f;
+        y[3] += v.w * f;
+    }
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    const int64_t row = (b * Tq + qi) * Hq + h;
+    *(uint2 *)(o + row * D + c) =
+        make_uint2(pack2<DT>(y[0] * inv, y[1] * inv), pack2<DT>(y[2] * inv, y[3] * inv));
+    if (c == 0)
+        lse[row] = l > 0.f ? (float)((double)mc * 0.6931471805599453 + log((double)l)) : -INFINITY;
 }
 
 // Whether the 16-bit kernels' buffer loads reach `rows` rows of `x` (a row every x.t elements,
@@ -371,35 +467,132 @@ extern "C" int dm_debug_trace_fwd(void *host, size_t bytes) {
 }
 #endif
 
+// How a call is split along the keys, and the bytes that takes (0: not split).
+//
+// Work items of 256 queries (128 at width 256) of one head are one a compute unit (two at width 64,
+// which run little faster together than one after the other), so a call of fewer than 256 lasts as
+// long as its longest: 96 key tiles of 64 for the last of 6144 causal queries, where the chip's share
+// is 36. Of the segment lengths that cut the longest item in up to 16, the one is taken whose
+// workgroups, laid on 256 compute units longest first, end earliest, each workgroup costing
+// kSegCost tiles besides its own (its start, its partial outputs) and the split kMergeCost (the
+// merge). Measured, before and after: 6144 causal queries of 8 heads, width 64: 125 -> 75 us; width 128, 2048
+// queries: 58 -> 35, 4096: 108 -> 65, 6144: 155 -> 110; width 256, 2048: 92 -> 56; 16 queries against 8192
+// keys of 8 heads of 128: 152 -> 28; unmasked 6144 of width 64 (192 equal items) are as fast whole.
+static size_t fwd_split(const dm_attention_desc *d, char *base, FwdSplit *sp) {
+    constexpr int kCUs = 256, kMinTiles = 6, kSegCost = 3, kMergeCost = 4;
+    const int64_t per = 32 * (d->d == 256 ? fwd_waves<256>() : fwd_waves<128>());
+    const int64_t nt = (d->tq + per - 1) / per, rows = d->hq * d->b;
+    sp->nseg = 0;
+    if (nt * rows == 0 || nt * rows >= kCUs || d->tk <= kMinTiles * kFwdN) return 0;
+    // key tiles of each query tile, from the mask's closed form (offsets lie on the device: packed
+    // sequences are taken for one)
+    MaskInfo m = mask_info(d);
+    m.kind = DM_MASK_NONE;
+    const int ntiles = (int)nt;
+    int n[kSplitTiles], most = 0;
+    for (int t = 0; t < ntiles; t++) {
+        int64_t lo, hi, x;
+        const int64_t q0 = (ntiles - 1 - t) * per;
+        row_bounds(m, q0, &lo, &x);
+        row_bounds(m, std::min(q0 + per, d->tq) - 1, &x, &hi);
+        n[t] = (int)std::max<int64_t>((hi - lo + kFwdN - 1) / kFwdN, 1);
+        most = std::max(most, n[t]);
+    }
+    // the time, in tiles, of segments of at most `steps`
+    auto ends = [&](int steps) -> int64_t {
+        std::pair<int, int64_t> len[kSplitTiles];  // length, how many
+        int64_t count = 0, total = 0;
+        for (int t = 0; t < ntiles; t++) {
+            const int ns = (n[t] + steps - 1) / steps;
+            len[t] = {(n[t] + ns - 1) / ns + kSegCost, ns * rows};
+            count += len[t].second;
+            total += len[t].second * len[t].first;
+        }
+        if (count > 2 * kCUs) return total / kCUs + steps / 4;
+        std::sort(len, len + ntiles, [](auto &a, auto &b) { return a.first > b.first; });
+        int64_t worst = len[0].first, at = count - 1;
+        // past a workgroup a unit, the k-th longest of the rest joins the k-th shortest of the first
+        int i = 0, j = ntiles - 1;
+        int64_t ci = len[0].second, cj = count - len[ntiles - 1].second;
+        for (int64_t k = 2 * kCUs - count; k < kCUs; k++) {
+            while (k >= ci) ci += len[++i].second;
+            while (at < cj) cj -= len[--j].second;
+            worst = std::max<int64_t>(worst, len[i].first + len[j].first);
+            at--;
+        }
+        return worst;
+    };
+    int best = most;
+    int64_t least = ends(most) * 7 / 8 - kMergeCost;  // an eighth to gain, or whole
+    for (int k = 2; k <= 16; k++) {
+        const int s = (most + k - 1) / k;
+        if (s < kMinTiles) break;
+        const int64_t e = ends(s);
+        if (e < least) least = e, best = s;
+    }
+    int c = 0;
+    for (int t = 0; t < ntiles; t++) {
+        sp->first[t] = (uint16_t)c;
+        c += (n[t] + best - 1) / best;
+    }
+    sp->first[ntiles] = (uint16_t)c;
+    if (c == ntiles) return 0;
+    sp->nseg = c;
+    const size_t on = align_up((size_t)(c * rows * per * d->d) * 4);
+    sp->o = (float *)base;
+    sp->ml = (float2 *)(base + on);
+    return on + align_up((size_t)(c * rows * per) * 8);
+}
+
+size_t mfma_fwd_workspace(const dm_attention_desc *d) {
+    FwdSplit sp;
+    const bool shape = (d->dtype == DM_BF16 || d->dtype == DM_F16) && (d->d == 64 || d->d == 128 || d->d == 256);
+    return shape ? fwd_split(d, nullptr, &sp) : 0;
+}
+
 int launch_attn_fwd_mfma(const MaskInfo &m, const dm_attention_desc *d, float scale,
                          const void *q, const void *k, const void *v, void *o, float *lse,
-                         hipStream_t st) {
+                         void *workspace, size_t workspace_bytes, hipStream_t st) {
     const int nw = d->d == 256 ? fwd_waves<256>() : fwd_waves<128>();
     const int64_t per = 32 * nw;  // queries per workgroup
     const int64_t ntiles = (d->tq + per - 1) / per;
     const int64_t nwork = ntiles * d->hq * d->b;
     const int64_t nblocks = (nwork + 7) / 8 * 8;
     if (nblocks >= (1ll << 31)) return refuse("attention: too many query tiles");
-    dim3 grid((unsigned)nblocks), block(64 * nw);
+    // a caller without the workspace gets the call in one piece
+    FwdSplit sp;
+    const size_t need = fwd_split(d, (char *)workspace, &sp);
+    const bool split = need && workspace && workspace_bytes >= need && aligned_16b(workspace);
+    const int64_t nwg = split ? sp.nseg * d->hq * d->b : nblocks;
+    dim3 grid((unsigned)nwg), block(64 * nw);
     const uint16_t *qq = (const uint16_t *)q, *kk = (const uint16_t *)k, *vv = (const uint16_t *)v;
     uint16_t *oo = (uint16_t *)o;
     const AttnStrides sd = attn_strides(d);
-#define FWD(DT, DD)                                                                           \
-    if (m.pad)                                                                                \
-        attn_fwd_mfma<DT, DD, true><<<grid, block, 0, st>>>(m, d->b, d->hq, d->hkv, scale, sd,  \
-                                                          qq, kk, vv, oo, lse);              \
-    else                                                                                      \
-        attn_fwd_mfma<DT, DD, false><<<grid, block, 0, st>>>(m, d->b, d->hq, d->hkv, scale, sd, \
-                                                           qq, kk, vv, oo, lse)
+#define FWD1(DT, DD, PAD, SPLIT)                                                                  \
+    attn_fwd_mfma<DT, DD, PAD, SPLIT><<<grid, block, 0, st>>>(m, d->b, d->hq, d->hkv, scale, sd, qq, \
+                                                              kk, vv, oo, lse, sp)
+#define FWD(DT, DD)                                                                                   \
+    {                                                                                                 \
+        if (split) {                                                                                  \
+            if (m.pad) FWD1(DT, DD, true, true); else FWD1(DT, DD, false, true);                      \
+            attn_fwd_merge<DT, DD><<<dim3((unsigned)nwork, (unsigned)(per * DD / 1024)), 256, 0, st>>>( \
+                d->tq, d->hq, d->hkv, d->b, (int)ntiles, sp, oo, lse);                                           \
+        } else if (m.pad) {                                                                           \
+            FWD1(DT, DD, true, false);                                                                \
+        } else {                                                                                      \
+            FWD1(DT, DD, false, false);                                                               \
+        }                                                                                             \
+    }
     {
         KernelTimer timer(DM_KERNEL_ATTN_FWD, st);
         if (d->dtype == DM_BF16) {
-            if (d->d == 64) { FWD(DM_BF16, 64); } else if (d->d == 128) { FWD(DM_BF16, 128); } else { FWD(DM_BF16, 256); }
+            if (d->d == 64) FWD(DM_BF16, 64) else if (d->d == 128) FWD(DM_BF16, 128) else FWD(DM_BF16, 256)
         } else {
-            if (d->d == 64) { FWD(DM_F16, 64); } else if (d->d == 128) { FWD(DM_F16, 128); } else { FWD(DM_F16, 256); }
+            if (d->d == 64) FWD(DM_F16, 64) else if (d->d == 128) FWD(DM_F16, 128) else FWD(DM_F16, 256)
         }
     }
 #undef FWD
+#undef FWD1
     probe_add(DM_PROBE_ATTN_FWD_MFMA);
     DM_LAUNCH_CHECK("attention: MFMA forward launch");
     return DM_OK;

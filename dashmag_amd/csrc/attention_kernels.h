@@ -25,7 +25,8 @@ bool rows_fit_32bit(const Strd &x, int64_t rows, int64_t d);
 bool mfma_fwd_takes(const dm_attention_desc *d, const void *q, const void *k, const void *v);
 int launch_attn_fwd_mfma(const MaskInfo &m, const dm_attention_desc *d, float scale,
                          const void *q, const void *k, const void *v, void *o, float *lse,
-                         hipStream_t st);
+                         void *workspace, size_t workspace_bytes, hipStream_t st);
+size_t mfma_fwd_workspace(const dm_attention_desc *d);
 bool mfma_bwd_takes(const dm_attention_desc *d, const void *q, const void *k, const void *v,
                     const void *o, const void *d_o);
 size_t mfma_bwd_workspace(const dm_attention_desc *d);

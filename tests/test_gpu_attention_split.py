@@ -1,0 +1,58 @@
+"""The 16-bit forward split along the keys (calls of fewer work items than compute units) against
+the f64 oracle: segments that divide the key tiles unevenly, query tiles of one segment beside
+tiles of several, rows that see no key, windows, key padding, cross lengths, a batch, packed
+sequences, and few queries against many keys; and the same call in one piece, through the C ABI
+without a workspace. Bounds as test_gpu_attention_sweep.py."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+import dashmag_amd as dm
+import oracle
+from conformance import BF16, F16
+from dashmag_amd import _lib, ops
+from fixtures import errors
+from test_gpu_attention_sweep import U, _build, host
+
+pytestmark = pytest.mark.gpu
+
+# (name, B, Tq, Tk, Hq, Hkv, mask spec, causal, window, scale)
+CASES = [
+    ("causal_1300", 1, 1300, 1300, 2, 1, None, True, None, None),
+    ("none_16x3000", 1, 16, 3000, 4, 2, None, False, None, None),
+    ("causal_cross_700x2100_b2", 2, 700, 2100, 2, 1, None, True, None, 0.2),
+    ("causal_empty_rows_1800x1500", 1, 1800, 1500, 2, 2, None, True, None, None),
+    ("window_1800", 1, 1800, 1800, 2, 1, None, True, (1000, U), None),
+    ("padding_1700_b3", 3, 1700, 1700, 1, 1, "padding", False, None, None),
+    ("packed_1700", 1, None, None, 2, 1, ("packed", [1500, 0, 200], [1500, 0, 200], 30), True, None,
+     None),
+]
+
+
+@pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 64), (torch.bfloat16, 128), (torch.float16, 128),
+                                     (torch.bfloat16, 256)])
+@pytest.mark.parametrize("case", CASES, ids=[c[0] for c in CASES])
+def test_split_matches_oracle(case, dtype, d):
+    print(f"case {case[0]} {dtype} D={d}", flush=True)
+    (q, k, v, _), mask, opts, mk = _build(case, dtype, d, 9000 + 17 * CASES.index(case) + d)
+    desc = ops._attention_desc("attention", q, k, v, mask, opts, keep := [])
+    lib = _lib.lib()
+    assert lib.dm_attention_fwd_workspace(ctypes.byref(desc)) > 0, "the call is not split"
+    _lib.probe_reset()
+    o, lse = dm.attention_with_lse(q, k, v, mask, opts)
+    o1, lse1 = torch.empty_like(o), torch.empty_like(lse)
+    rc = lib.dm_attention_fwd(ctypes.byref(desc), q.data_ptr(), k.data_ptr(), v.data_ptr(),
+                              o1.data_ptr(), lse1.data_ptr(), None, 0,
+                              torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, _lib.last_error()
+    torch.cuda.synchronize()
+    assert _lib.probe_counts()["attn_fwd_mfma"] == 2
+    eo, el = oracle.attention_fwd(mk(host(q), host(k), host(v)), "f64")
+    bounds = (BF16 if dtype == torch.bfloat16 else F16).masks
+    for go, gl in ((o, lse), (o1, lse1)):
+        ro, rl = errors(host(go), eo)[1], errors(host(gl), el)[1]
+        print(f"  o {ro:.2e} lse {rl:.2e}")
+        assert ro <= 2 * bounds[0] and rl <= 2 * bounds[1] * max(1.0, np.sqrt(k.shape[1] / 64))
+        assert np.all(host(go)[el == -np.inf] == 0.0)

@@ -54,6 +54,19 @@ __device__ __forceinline__ float lp_block_sum(float x, float *sm) {
     __syncthreads();
     return (sm[0] + sm[1]) + (sm[2] + sm[3]);
 }
+// Four sums at once (sm: 16 floats): one pair of barriers.
+__device__ __forceinline__ void lp_block_sum4(float (&x)[4], float *sm) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) x[i] = wave_sum(x[i]);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) sm[4 * i + (threadIdx.x >> 6)] = x[i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; i++) x[i] = (sm[4 * i] + sm[4 * i + 1]) + (sm[4 * i + 2] + sm[4 * i + 3]);
+}
 __device__ __forceinline__ float lp_block_max(float x, float *sm) {
     x = wave_max(x);
     const int w = threadIdx.x >> 6;
@@ -87,31 +100,43 @@ __global__ __launch_bounds__(kLpThreads) void lp_stats(int64_t rows, int64_t cw,
                                                        float *__restrict__ st, int64_t nst,
                                                        void *__restrict__ E, void *__restrict__ E2,
                                                        float *__restrict__ o) {
-    __shared__ float sm[4];
+    __shared__ float sm[16];
     const int64_t row = blockIdx.x;
     if (row >= rows) return;
     const float *z = Z + row * cw;
     const bool vec = (cw & 3) == 0;
     float x[NV][4];
+    // (read with the logits, used after them)
+    const float m = st[LP_M * nst + row];
+    const float s_old = st[LP_S * nst + row], a_old = st[LP_A * nst + row];
+    const float r_old = st[LP_R * nst + row];
+    const int64_t t = targets[row];
+    // every load first: a row of 8192 logits is 8 of them a thread in flight at once
+    uint32_t mw[NV];
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+        const int64_t j = 4 * (int64_t)threadIdx.x + 1024 * i;
+        if (vec) {
+            const float4 v = j < cw ? *(const float4 *)(z + j) : make_float4(-FLT_MAX, -FLT_MAX, -FLT_MAX, -FLT_MAX);
+            x[i][0] = v.x, x[i][1] = v.y, x[i][2] = v.z, x[i][3] = v.w;
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; q++) x[i][q] = j + q < cw ? z[j + q] : -FLT_MAX;
+        }
+        mw[i] = j < cw ? bits[(c0 + j) >> 5] : 0;
+    }
     uint32_t live = 0;  // bit 4 i + q: column 4 t + 1024 i + q is in the chunk and unmasked
     // the chunk's maximum over the unmasked tokens
     float mx = -FLT_MAX;
 #pragma unroll
     for (int i = 0; i < NV; i++) {
         const int64_t j = 4 * (int64_t)threadIdx.x + 1024 * i;
-        if (vec && j < cw) {
-            const float4 v = *(const float4 *)(z + j);
-            x[i][0] = v.x, x[i][1] = v.y, x[i][2] = v.z, x[i][3] = v.w;
-        } else {
-#pragma unroll
-            for (int q = 0; q < 4; q++) x[i][q] = j + q < cw ? z[j + q] : -FLT_MAX;
-        }
         // the masked bits of the 4 columns: one word when they share it
         const int64_t tok = c0 + j;
         uint32_t mb = 0;
         if (j < cw) {
             if ((tok & 31) <= 28) {
-                mb = bits[tok >> 5] >> (tok & 31);
+                mb = mw[i] >> (tok & 31);
             } else {
 #pragma unroll
                 for (int q = 0; q < 4; q++)
@@ -126,14 +151,8 @@ __global__ __launch_bounds__(kLpThreads) void lp_stats(int64_t rows, int64_t cw,
             }
     }
     mx = lp_block_max(mx, sm);
-    // this row's running state, read by every thread before the block reductions below (thread
-    // 0 rewrites it after them)
-    const float m = st[LP_M * nst + row];
-    const float s_old = st[LP_S * nst + row], a_old = st[LP_A * nst + row];
-    const float r_old = st[LP_R * nst + row];
     const float m_new = mx > m ? mx : m;
     const float shift = m - m_new, alpha = expf(shift);
-    const int64_t t = targets[row];
     const int64_t tl = t - c0;
     const bool has_t = tl >= 0 && tl < cw && !lp_masked(bits, t);
     // the chunk's sums; the weights of the next product (0 for the target and masked tokens)
@@ -183,10 +202,9 @@ __global__ __launch_bounds__(kLpThreads) void lp_stats(int64_t rows, int64_t cw,
             }
         }
     }
-    se = lp_block_sum(se, sm);
-    sz = lp_block_sum(sz, sm);
-    sa = lp_block_sum(sa, sm);
-    sr = lp_block_sum(sr, sm);
+    float sums[4] = {se, sz, sa, sr};
+    lp_block_sum4(sums, sm);
+    se = sums[0], sz = sums[1], sa = sums[2], sr = sums[3];
     if constexpr (EK != 0) {
         // o is still zero while nothing has been summed (the first chunk)
         if (alpha != 1.f && s_old != 0.f)
@@ -308,7 +326,10 @@ __global__ void lce_coef(int64_t n, const float *__restrict__ rows,
 
 // The logits' gradient of a chunk (logprob/reference.rs:345-366): g = e^{z - lse}(A - E (z - lse))
 // + C, T + C at the target, 0 at a masked id; written as bf16 (BF = true, the products' operand,
-// as torch's bf16 linear layer rounds its output's gradient) or f32. One row per workgroup.
+// as torch's bf16 linear layer rounds its output's gradient) or f32. One row per workgroup, 8
+// columns a thread in 16-byte pieces where the chunk's width allows, a row's loads all in flight
+// before the first exponential (an element a thread at a time, 2048 rows of 8192 took 34 us, at
+// 2.9 TB/s).
 template <bool BF>
 __global__ __launch_bounds__(kLpThreads) void lce_dz(int64_t rows, int64_t cw, int64_t c0,
                                                      const float *__restrict__ Z,
@@ -323,16 +344,46 @@ __global__ __launch_bounds__(kLpThreads) void lce_dz(int64_t rows, int64_t cw, i
     const float T = coef[LC_T * n + row], E = coef[LC_E * n + row], C = coef[LC_C * n + row];
     const int64_t tl = targets[row] - c0;
     const float *z = Z + row * cw;
-    for (int64_t j = threadIdx.x; j < cw; j += kLpThreads) {
-        float g;
-        if (lp_masked(bits, c0 + j)) {
-            g = 0.f;
-        } else if (j == tl) {
-            g = T;
-        } else {
-            const float dz = z[j] - lse;
-            g = expf(dz) * (A - E * dz) + C;
+    auto grad = [&](float x, bool masked, int64_t j) {
+        const float dz = x - lse;
+        const float g = expf(dz) * (A - E * dz) + C;
+        return masked ? 0.f : j == tl ? T : g;
+    };
+    if (cw % 8 == 0 && c0 % 8 == 0) {
+        constexpr int NB = (int)(kLpMaxChunk / (8 * kLpThreads));
+        float4 x[NB][2];
+        uint32_t mw[NB];
+#pragma unroll
+        for (int i = 0; i < NB; i++) {
+            const int64_t j = 8 * ((int64_t)threadIdx.x + kLpThreads * i);
+            if (j < cw) {
+                x[i][0] = *(const float4 *)(z + j);
+                x[i][1] = *(const float4 *)(z + j + 4);
+                mw[i] = bits[(c0 + j) >> 5] >> ((c0 + j) & 31);
+            }
         }
+#pragma unroll
+        for (int i = 0; i < NB; i++) {
+            const int64_t j = 8 * ((int64_t)threadIdx.x + kLpThreads * i);
+            if (j >= cw) break;
+            const float v[8] = {x[i][0].x, x[i][0].y, x[i][0].z, x[i][0].w,
+                                x[i][1].x, x[i][1].y, x[i][1].z, x[i][1].w};
+            float g[8];
+#pragma unroll
+            for (int q = 0; q < 8; q++) g[q] = grad(v[q], (mw[i] >> q) & 1u, j + q);
+            if constexpr (BF) {
+                *(uint4 *)((uint16_t *)G + row * cw + j) =
+                    make_uint4(pack2<DM_BF16>(g[0], g[1]), pack2<DM_BF16>(g[2], g[3]),
+                               pack2<DM_BF16>(g[4], g[5]), pack2<DM_BF16>(g[6], g[7]));
+            } else {
+                *(float4 *)((float *)G + row * cw + j) = make_float4(g[0], g[1], g[2], g[3]);
+                *(float4 *)((float *)G + row * cw + j + 4) = make_float4(g[4], g[5], g[6], g[7]);
+            }
+        }
+        return;
+    }
+    for (int64_t j = threadIdx.x; j < cw; j += kLpThreads) {
+        const float g = grad(z[j], lp_masked(bits, c0 + j), j);
         if constexpr (BF)
             ((uint16_t *)G)[row * cw + j] = f32_to_bf16(g);
         else
@@ -340,7 +391,6 @@ __global__ __launch_bounds__(kLpThreads) void lce_dz(int64_t rows, int64_t cw, i
     }
 }
 
-// f32 -> the dtype (a copy for f32), and fills with zeros.
 // f32 -> the dtype, 8 elements a thread per pass (two 16-byte loads, one 16-byte store for a
 // 16-bit dtype); the tail past a multiple of 8 element by element.
 __global__ void lp_cast(int64_t count, const float *__restrict__ x, void *__restrict__ y, int dt) {
@@ -367,11 +417,6 @@ __global__ void lp_cast(int64_t count, const float *__restrict__ x, void *__rest
     for (int64_t i = 8 * n8 + (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count;
          i += stride)
         st_any(dt, y, i, x[i]);
-}
-__global__ void lp_zero(int64_t count, float *__restrict__ x) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count;
-         i += (int64_t)gridDim.x * blockDim.x)
-        x[i] = 0.f;
 }
 __global__ void lp_widen16(int64_t count, const _Float16 *__restrict__ x, float *__restrict__ y) {
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count;
@@ -403,11 +448,12 @@ static hipblasLtHandle_t lt_handle() {
     return it->second;
 }
 
-// Column-major D (m x n, ld m) = op(A) op(B) + beta D, f32 out, f32 accumulation; A and B of
+// Column-major D (m x n, ld m) = op(A) op(B) + beta D, of type `td`, f32 accumulation; A and B of
 // type `t`, A stored m x k (ta = N, lda m) or k x m (ta = T, lda k), B stored k x n (tb = N,
 // ldb k) or n x k (tb = T, ldb n).
 static int lt_gemm(hipStream_t st, bool ta, bool tb, int64_t m, int64_t n, int64_t k,
-                   const void *A, const void *B, hipDataType t, float beta, float *Dm, void *ws) {
+                   const void *A, const void *B, hipDataType t, float beta, void *Dm, void *ws,
+                   hipDataType td = HIP_R_32F) {
     hipblasLtHandle_t h = lt_handle();
     if (!h) {
         set_error("no hipBLASLt handle");
@@ -416,7 +462,7 @@ static int lt_gemm(hipStream_t st, bool ta, bool tb, int64_t m, int64_t n, int64
     int dev = 0;
     (void)hipGetDevice(&dev);
     thread_local std::map<std::vector<int64_t>, LtGemm> cache;
-    const std::vector<int64_t> key{dev, ta, tb, m, n, k, (int64_t)t, beta != 0.f};
+    const std::vector<int64_t> key{dev, ta, tb, m, n, k, (int64_t)t, beta != 0.f, (int64_t)td};
     LtGemm &g = cache[key];
     if (!g.desc) {
         const hipblasOperation_t opa = ta ? HIPBLAS_OP_T : HIPBLAS_OP_N;
@@ -429,7 +475,7 @@ static int lt_gemm(hipStream_t st, bool ta, bool tb, int64_t m, int64_t n, int64
         good = good && hipblasLtMatrixLayoutCreate(&g.a, t, ta ? k : m, ta ? m : k, ta ? k : m) == HIPBLAS_STATUS_SUCCESS;
         good = good && hipblasLtMatrixLayoutCreate(&g.b, t, tb ? n : k, tb ? k : n, tb ? n : k) ==
                            HIPBLAS_STATUS_SUCCESS;
-        good = good && hipblasLtMatrixLayoutCreate(&g.c, HIP_R_32F, m, n, m) == HIPBLAS_STATUS_SUCCESS;
+        good = good && hipblasLtMatrixLayoutCreate(&g.c, td, m, n, m) == HIPBLAS_STATUS_SUCCESS;
         hipblasLtMatmulPreference_t pref = nullptr;
         good = good && hipblasLtMatmulPreferenceCreate(&pref) == HIPBLAS_STATUS_SUCCESS;
         const uint64_t wsb = kLtWorkspace;
@@ -458,16 +504,21 @@ static int lt_gemm(hipStream_t st, bool ta, bool tb, int64_t m, int64_t n, int64
     return DM_OK;
 }
 
+// Rows of the loss's backward whose chunk of logits' gradients is held for one weight-gradient
+// product (at 8192 columns in bf16 256 MB at most).
+constexpr int64_t kLceGroup = 16384;
+
 struct LpPlan {
     int64_t block, chunk;  // rows per block, vocabulary tokens per chunk
+    int64_t group;         // rows (whole blocks) whose logits' gradients are held at once
     bool bf16;             // both operands bf16 (else both taken as f32)
     size_t off_bits, off_state, off_z, off_e, off_h, off_w, off_lt, off_coef, off_gh, off_gw;
     size_t total;
 };
 
 // What a call holds: grad (the log-probability's softmax weights, two bf16 parts or f32),
-// dz (the loss's logits gradient, bf16 or f32), and the loss's f32 gradient accumulators when
-// the gradients' dtype is not f32.
+// dz (the loss's logits gradient of a group of row blocks, bf16 or f32), and the loss's f32 gradient
+// accumulators when the gradients' dtype is not f32: the hidden's, and a chunk of the weight's.
 static LpPlan lp_plan(const dm_logprob_desc *d, bool grad, bool dz, bool gh32, bool gw32) {
     LpPlan p{};
     const int64_t nb = d->n > 0 ? (d->n + d->row_chunk - 1) / d->row_chunk : 1;
@@ -477,6 +528,8 @@ static LpPlan lp_plan(const dm_logprob_desc *d, bool grad, bool dz, bool gh32, b
     p.chunk = d->vocab_chunk > 0 ? d->vocab_chunk : kLpMaxChunk;
     p.chunk = std::min<int64_t>({p.chunk, kLpMaxChunk, std::max<int64_t>(d->v, 1)});
     p.bf16 = d->hidden_dtype == DM_BF16 && d->weight_dtype == DM_BF16;
+    p.group = std::max<int64_t>(1, kLceGroup / p.block) * p.block;
+    p.group = std::min(p.group, std::max<int64_t>(d->n, 1));
     const int64_t n1 = std::max<int64_t>(d->n, 1);
     size_t o = 0;
     p.off_bits = o;
@@ -486,7 +539,8 @@ static LpPlan lp_plan(const dm_logprob_desc *d, bool grad, bool dz, bool gh32, b
     p.off_z = o;
     o += align_up((size_t)p.block * p.chunk * 4);
     p.off_e = o;
-    if (grad || dz) o += align_up((size_t)p.block * p.chunk * 4) + 256;
+    if (grad) o += align_up((size_t)p.block * p.chunk * 4) + 256;
+    if (dz) o += align_up((size_t)p.group * p.chunk * (p.bf16 ? 2 : 4));
     p.off_h = o;
     if (!p.bf16 && d->hidden_dtype != DM_F32) o += align_up((size_t)d->n * d->d * 4);
     p.off_w = o;
@@ -496,7 +550,7 @@ static LpPlan lp_plan(const dm_logprob_desc *d, bool grad, bool dz, bool gh32, b
     p.off_gh = o;
     if (gh32) o += align_up((size_t)d->n * d->d * 4);
     p.off_gw = o;
-    if (gw32) o += align_up((size_t)d->v * d->d * 4);
+    if (gw32) o += align_up((size_t)p.chunk * d->d * 4);
     p.off_lt = o;
     o += kLtWorkspace;
     p.total = o;
@@ -771,18 +825,9 @@ int dm_linear_cross_entropy_bwd(const dm_lce_desc *d, const void *hidden, const 
     hipStream_t st = (hipStream_t)stream;
     char *ws = (char *)workspace;
     float *gh = grad_hidden ? (f32 ? (float *)grad_hidden : (float *)(ws + p.off_gh)) : nullptr;
-    float *gw = grad_weight ? (f32 ? (float *)grad_weight : (float *)(ws + p.off_gw)) : nullptr;
-    // (the accumulators need no clearing: the first row block's products write grad_weight and
-    // each row block's first chunk writes its rows of grad_hidden, with beta = 0)
     if (lp->n == 0) {
-        if (gw) {
-            lp_zero<<<1024, 256, 0, st>>>(lp->v * lp->d, gw);
-            DM_LAUNCH_CHECK("linear_cross_entropy: zero");
-        }
-        if (grad_weight && !f32) {
-            lp_cast<<<1024, 256, 0, st>>>(lp->v * lp->d, gw, grad_weight, lp->weight_dtype);
-            DM_LAUNCH_CHECK("linear_cross_entropy: cast");
-        }
+        if (grad_weight) fill_zero(grad_weight, (size_t)lp->v * lp->d * dtype_bytes(lp->weight_dtype), st);
+        DM_LAUNCH_CHECK("linear_cross_entropy: zero");
         return DM_OK;
     }
     if (int rc = lp_upload_bits(bits, ws, p, st)) return rc;
@@ -793,46 +838,63 @@ int dm_linear_cross_entropy_bwd(const dm_lce_desc *d, const void *hidden, const 
     lce_coef<<<(unsigned)((lp->n + 255) / 256), 256, 0, st>>>(
         lp->n, rows, upstream, d->label_smoothing, d->z_loss, inv_classes, d->entropy, coef);
     DM_LAUNCH_CHECK("linear_cross_entropy: coefficients");
-    // the gradient pass (logprob/reference.rs:289-380): the logits again, the logits' gradient,
-    // then grad_hidden_b += G W_c and grad_weight_c += G^T H_b
+    // The gradient pass (logprob/reference.rs:289-380), per vocabulary chunk: the logits again and
+    // their gradient, a block of rows after another into G [rows of the group, chunk]; then
+    // grad_hidden += G W_c, and grad_weight_c = G^T H over all of the group's rows in one product.
+    // The chunk is the outer loop so that the weight's gradient is summed within a product and
+    // written once, in its own dtype (bf16 with at most one group of rows): accumulated per row
+    // block in f32 over the whole vocabulary, 4096 rows of 4096 by 151936 tokens moved 10 GB more
+    // (of which 3.7 GB, 720 us, rounded the sum), and its products of 2048 rows each took 165 us a
+    // chunk where one of 4096 takes 240. With more groups an f32 chunk accumulates.
+    // The first product of each accumulator runs with beta = 0, which hipBLASLt takes as "C is not
+    // read" (the accumulators are never cleared; a workspace poisoned with NaN gives the same bits
+    // as a zeroed one, a property the GPU tests hold it to).
     float *Z = (float *)(ws + p.off_z);
     void *G = ws + p.off_e, *lt_ws = ws + p.off_lt;
     const hipDataType op_t = p.bf16 ? HIP_R_16BF : HIP_R_32F;
-    const size_t esz = p.bf16 ? 2 : 4;
+    const size_t esz = p.bf16 ? 2 : 4, wsz = dtype_bytes(lp->weight_dtype);
     const uint32_t *dbits = (const uint32_t *)(ws + p.off_bits);
-    for (int64_t r0 = 0; r0 < lp->n; r0 += p.block) {
-        const int64_t rows_b = std::min<int64_t>(p.block, lp->n - r0);
-        for (int64_t c0 = 0; c0 < lp->v; c0 += p.chunk) {
-            const int64_t cw = std::min<int64_t>(p.chunk, lp->v - c0);
-            if (int rc = lp_logits(lp, p, H, W, r0, rows_b, c0, cw, Z, lt_ws, st)) return rc;
-            if (p.bf16)
-                lce_dz<true><<<(unsigned)rows_b, kLpThreads, 0, st>>>(
-                    rows_b, cw, c0, Z, targets + r0, dbits, rows + r0, coef + r0, lp->n, G);
-            else
-                lce_dz<false><<<(unsigned)rows_b, kLpThreads, 0, st>>>(
-                    rows_b, cw, c0, Z, targets + r0, dbits, rows + r0, coef + r0, lp->n, G);
-            DM_LAUNCH_CHECK("linear_cross_entropy: logits gradient");
-            const char *Wc = (const char *)W + (size_t)c0 * lp->d * esz;
-            // grad_hidden (column-major D x rows) += W_c as stored (D x cw) G^T (cw x rows).
-            // The first product of each accumulator runs with beta = 0, which hipBLASLt takes
-            // as "C is not read" (the accumulators are never cleared; a workspace poisoned with
-            // NaN gives the same bits as a zeroed one, a property the GPU tests hold it to)
+    const bool direct = f32 || (p.bf16 && p.group >= lp->n && aligned_16b(grad_weight));
+    for (int64_t c0 = 0; c0 < lp->v; c0 += p.chunk) {
+        const int64_t cw = std::min<int64_t>(p.chunk, lp->v - c0);
+        const char *Wc = (const char *)W + (size_t)c0 * lp->d * esz;
+        char *gwc = grad_weight ? (char *)grad_weight + (size_t)c0 * lp->d * wsz : nullptr;
+        float *gw = (float *)(ws + p.off_gw);  // the f32 chunk, where the product can't write gwc
+        for (int64_t g0 = 0; g0 < lp->n; g0 += p.group) {
+            const int64_t rows_g = std::min<int64_t>(p.group, lp->n - g0);
+            for (int64_t r0 = g0; r0 < g0 + rows_g; r0 += p.block) {
+                const int64_t rows_b = std::min<int64_t>(p.block, g0 + rows_g - r0);
+                void *Gb = (char *)G + (size_t)(r0 - g0) * cw * esz;
+                if (int rc = lp_logits(lp, p, H, W, r0, rows_b, c0, cw, Z, lt_ws, st)) return rc;
+                if (p.bf16)
+                    lce_dz<true><<<(unsigned)rows_b, kLpThreads, 0, st>>>(
+                        rows_b, cw, c0, Z, targets + r0, dbits, rows + r0, coef + r0, lp->n, Gb);
+                else
+                    lce_dz<false><<<(unsigned)rows_b, kLpThreads, 0, st>>>(
+                        rows_b, cw, c0, Z, targets + r0, dbits, rows + r0, coef + r0, lp->n, Gb);
+                DM_LAUNCH_CHECK("linear_cross_entropy: logits gradient");
+            }
+            // grad_hidden (column-major D x rows) += W_c as stored (D x cw) G^T (cw x rows)
             if (gh)
-                if (int rc = lt_gemm(st, false, false, lp->d, rows_b, cw, Wc, G, op_t,
-                                     c0 == 0 ? 0.f : 1.f, gh + r0 * lp->d, lt_ws))
+                if (int rc = lt_gemm(st, false, false, lp->d, rows_g, cw, Wc, G, op_t,
+                                     c0 == 0 ? 0.f : 1.f, gh + g0 * lp->d, lt_ws))
                     return rc;
-            // grad_weight_c (column-major D x cw) += H_b as stored (D x rows) G (rows x cw; G
-            // is stored cw x rows, so op(B) = T)
-            if (gw)
-                if (int rc = lt_gemm(st, false, true, lp->d, cw, rows_b,
-                                     (const char *)H + (size_t)r0 * lp->d * esz, G, op_t,
-                                     r0 == 0 ? 0.f : 1.f, gw + c0 * lp->d, lt_ws))
+            // grad_weight_c (column-major D x cw) += H as stored (D x rows) G (rows x cw; G is
+            // stored cw x rows, so op(B) = T)
+            if (gwc)
+                if (int rc = lt_gemm(st, false, true, lp->d, cw, rows_g,
+                                     (const char *)H + (size_t)g0 * lp->d * esz, G, op_t,
+                                     g0 == 0 ? 0.f : 1.f, direct ? (void *)gwc : gw, lt_ws,
+                                     direct && !f32 ? HIP_R_16BF : HIP_R_32F))
                     return rc;
         }
+        if (gwc && !direct) {
+            lp_cast<<<1024, 256, 0, st>>>(cw * lp->d, gw, gwc, lp->weight_dtype);
+            DM_LAUNCH_CHECK("linear_cross_entropy: cast");
+        }
     }
-    if (!f32) {
-        if (grad_hidden) lp_cast<<<1024, 256, 0, st>>>(lp->n * lp->d, gh, grad_hidden, lp->hidden_dtype);
-        if (grad_weight) lp_cast<<<1024, 256, 0, st>>>(lp->v * lp->d, gw, grad_weight, lp->weight_dtype);
+    if (!f32 && grad_hidden) {
+        lp_cast<<<1024, 256, 0, st>>>(lp->n * lp->d, gh, grad_hidden, lp->hidden_dtype);
         DM_LAUNCH_CHECK("linear_cross_entropy: cast");
     }
     probe_add(DM_PROBE_LCE_BWD);

@@ -22,33 +22,26 @@
 namespace dm {
 
 // ------------------------------------------------------------------------------------------
-// Plan (chunk/cube.rs:80-175): per sequence its first chunk, per chunk its sequence, first
-// token and token count. Packed sequences are chunked from their own first token; every chunk
-// index up to the host's bound n_max that no sequence uses gets a count of 0.
+// Plan (chunk/cube.rs:80-175) of packed sequences: per sequence its first chunk, per chunk its first
+// token and token count. Sequences are chunked from their own first token; every chunk index up to
+// the host's bound n_max that no sequence uses gets a count of 0. A batch without offsets needs no
+// plan: GdrPlan has it in closed form.
 // ------------------------------------------------------------------------------------------
 
 __global__ __launch_bounds__(1024) void gdr_plan(int64_t nseq, int64_t T, int64_t n_max,
-                                                 const int32_t *__restrict__ cu,
-                                                 int32_t *__restrict__ seq_chunk0,
-                                                 int32_t *__restrict__ chunk_seq,
-                                                 int32_t *__restrict__ chunk_tok0,
-                                                 int32_t *__restrict__ chunk_len,
-                                                 int32_t *__restrict__ seq_order) {
+                                                 const int32_t *__restrict__ cu, GdrPlan p) {
+    int32_t *seq_chunk0 = p.seq_chunk0, *chunk_tok0 = p.chunk_tok0, *chunk_len = p.chunk_len,
+            *seq_order = p.seq_order;
     __shared__ int32_t part[1024];
     const int tid = threadIdx.x;
     const int64_t per = (nseq + 1023) / 1024;
     const int64_t s0 = tid * per, s1 = s0 + per < nseq ? s0 + per : nseq;
     auto span = [&](int64_t s, int64_t *a, int64_t *b) {
-        if (cu) {
-            *a = cu[s];
-            *b = cu[s + 1];
-            if (*a < 0) *a = 0;
-            if (*b > T) *b = T;  // malformed offsets stay inside the tokens (cube.rs:80-91)
-            if (*b < *a) *b = *a;
-        } else {
-            *a = s * T;
-            *b = s * T + T;
-        }
+        *a = cu[s];
+        *b = cu[s + 1];
+        if (*a < 0) *a = 0;
+        if (*b > T) *b = T;  // malformed offsets stay inside the tokens (cube.rs:80-91)
+        if (*b < *a) *b = *a;
     };
     // chunks per thread's sequences, then an inclusive scan over the threads
     int32_t local = 0;
@@ -75,27 +68,24 @@ __global__ __launch_bounds__(1024) void gdr_plan(int64_t nseq, int64_t T, int64_
     const int32_t used = part[1023] < n_max ? part[1023] : (int32_t)n_max;
     if (tid == 0) seq_chunk0[nseq] = used;
     __syncthreads();  // (orders the global writes above for the whole workgroup)
-    // optionally the sequences by chunk count, the most first (ties by index): the state
-    // passes start the longest chains first. Past kOrderMax sequences, the identity.
-    if (seq_order) {
-        for (int64_t s = tid; s < nseq; s += 1024) {
-            if (nseq > kOrderMax) {
-                seq_order[s] = (int32_t)s;
-                continue;
-            }
-            const int32_t n = seq_chunk0[s + 1] - seq_chunk0[s];
-            int32_t rank = 0;
-            for (int64_t u = 0; u < nseq; u++) {
-                const int32_t m = seq_chunk0[u + 1] - seq_chunk0[u];
-                rank += (m > n) | ((m == n) & (u < s));
-            }
-            seq_order[rank] = (int32_t)s;
+    // the sequences by chunk count, the most first (ties by index): the state passes start the
+    // longest chains first. Past kOrderMax sequences, the identity.
+    for (int64_t s = tid; s < nseq; s += 1024) {
+        if (nseq > kOrderMax) {
+            seq_order[s] = (int32_t)s;
+            continue;
         }
+        const int32_t n = seq_chunk0[s + 1] - seq_chunk0[s];
+        int32_t rank = 0;
+        for (int64_t u = 0; u < nseq; u++) {
+            const int32_t m = seq_chunk0[u + 1] - seq_chunk0[u];
+            rank += (m > n) | ((m == n) & (u < s));
+        }
+        seq_order[rank] = (int32_t)s;
     }
     // every chunk in parallel: its sequence is the last whose first chunk is at or before it
     for (int64_t x = tid; x < n_max; x += 1024) {
         if (x >= used) {
-            chunk_seq[x] = 0;
             chunk_tok0[x] = 0;
             chunk_len[x] = 0;
             continue;
@@ -111,7 +101,6 @@ __global__ __launch_bounds__(1024) void gdr_plan(int64_t nseq, int64_t T, int64_
         int64_t a, b;
         span(lo, &a, &b);
         const int64_t t = a + (x - seq_chunk0[lo]) * kChunk;
-        chunk_seq[x] = (int32_t)lo;
         chunk_tok0[x] = (int32_t)t;
         chunk_len[x] = (int32_t)(b - t < kChunk ? b - t : kChunk);
     }
@@ -313,9 +302,9 @@ __device__ __forceinline__ f32x4_t block16(const float *A, int lda, const float 
 template <int DT, bool BWD>
 __global__ __launch_bounds__(256) void gdr_prep(GdrArgs a, GdrWs w, const void *d_out) {
     const int64_t ch = blockIdx.x, n = ch / a.H, h = ch % a.H;
-    const int len = w.chunk_len[n];
+    const int len = w.plan.len(n);
     if (len == 0) return;
-    const int64_t tok0 = w.chunk_tok0[n];
+    const int64_t tok0 = w.plan.tok0(n);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int64_t Dk = a.Dk, Dv = a.Dv, KP = w.KP, VP = w.VP;
     __shared__ float4 smem[(2 * kPanels + 2 * kChunk * kMatS) / 4];
@@ -548,13 +537,13 @@ __global__ __launch_bounds__(256) void gdr_chain(GdrArgs a, GdrWs w, int64_t nsh
     // the column blocks of a (sequence, head) nshp (a multiple of 8) workgroups apart: on one XCD
     const int64_t slot = blockIdx.x % nshp;
     if (slot >= nsh) return;
-    const int64_t s = w.seq_order[slot / a.H], h = slot % a.H, sh = s * a.H + h;
+    const int64_t s = w.plan.order(slot / a.H), h = slot % a.H, sh = s * a.H + h;
     const int y0 = (int)(blockIdx.x / nshp) * 16 * NT;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int c = lane & 15, g4 = 4 * (lane >> 4);
     constexpr int KP = 64 * KTn, SS = KP + 4;
     const int64_t Dk = a.Dk, Dv = a.Dv, VP = w.VP;
-    const int c0 = w.seq_chunk0[s], c1 = w.seq_chunk0[s + 1];
+    const int c0 = w.plan.first(s), c1 = w.plan.first(s + 1);
     __shared__ float4 st4[16 * NT * SS / 4], vt4[16 * NT * kMatS / 4];
     float *St = (float *)st4, *Vt = (float *)vt4;
 
@@ -690,9 +679,9 @@ __global__ __launch_bounds__(256) void gdr_chain(GdrArgs a, GdrWs w, int64_t nsh
 template <int DT>
 __global__ __launch_bounds__(256) void gdr_output(GdrArgs a, GdrWs w, void *out) {
     const int64_t ch = blockIdx.x, n = ch / a.H, h = ch % a.H;
-    const int len = w.chunk_len[n];
+    const int len = w.plan.len(n);
     if (len == 0) return;
-    const int64_t tok0 = w.chunk_tok0[n], KP = w.KP, VP = w.VP;
+    const int64_t tok0 = w.plan.tok0(n), KP = w.KP, VP = w.VP;
     const int y0 = blockIdx.y * 64;
     __shared__ float4 smem[2 * kPanels / 4];
     __shared__ float gam[kChunk];
@@ -728,7 +717,7 @@ __global__ __launch_bounds__(256) void gdr_output(GdrArgs a, GdrWs w, void *out)
 // columns of dv_local = P^T dO, in the others a 64 x 64 tile of F = (gamma Q)^T dO; transposed.
 __global__ __launch_bounds__(256) void gdr_bwd_local(GdrArgs a, GdrWs w) {
     const int64_t ch = blockIdx.x, KP = w.KP, VP = w.VP;
-    if (w.chunk_len[ch / a.H] == 0) return;
+    if (w.plan.len(ch / a.H) == 0) return;
     const int vt = (int)(VP / 64), job = blockIdx.y;
     __shared__ float4 smem[2 * kPanels / 4];
     __shared__ float gam[kChunk];
@@ -760,7 +749,7 @@ __global__ __launch_bounds__(256) void gdr_bwd_local(GdrArgs a, GdrWs w) {
 // d_kt o K and the tile's part of sum(S o dS_next).
 __global__ __launch_bounds__(256) void gdr_bwd_states(GdrArgs a, GdrWs w) {
     const int64_t ch = blockIdx.x, KP = w.KP, VP = w.VP;
-    if (w.chunk_len[ch / a.H] == 0) return;
+    if (w.plan.len(ch / a.H) == 0) return;
     const int x0 = blockIdx.y * 64, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     __shared__ float4 smem[5 * kPanels / 4];
     __shared__ float gam[kChunk], lam[kChunk], red[2][2 * kChunk], sds[4];
@@ -839,7 +828,7 @@ __global__ __launch_bounds__(256) void gdr_bwd_states(GdrArgs a, GdrWs w) {
 // gradient from d_attn o P and dA o A (rows less columns).
 __global__ __launch_bounds__(256) void gdr_bwd_mats(GdrArgs a, GdrWs w) {
     const int64_t ch = blockIdx.x, n = ch / a.H, h = ch % a.H, KP = w.KP, VP = w.VP;
-    const int len = w.chunk_len[n];
+    const int len = w.plan.len(n);
     if (len == 0) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     __shared__ float4 smem[(2 * kPanels + 3 * kChunk * kMatS) / 4];
@@ -849,7 +838,7 @@ __global__ __launch_bounds__(256) void gdr_bwd_mats(GdrArgs a, GdrWs w) {
           *Dt = Ts + kChunk * kMatS;
     if (tid < kChunk) {
         G[tid] = w.G[ch * kChunk + tid];
-        bet[tid] = tid < len ? ld_any(a.beta_dt, a.beta, b_at(a, w.chunk_tok0[n] + tid, h)) : 0.f;
+        bet[tid] = tid < len ? ld_any(a.beta_dt, a.beta, b_at(a, w.plan.tok0(n) + tid, h)) : 0.f;
         bg[tid] = bet[tid] * expf((float)G[tid]);
     }
     const float *Tg = w.Tm + ch * kChunk * kChunk, *Pg = w.P + ch * kChunk * kChunk,
@@ -930,9 +919,9 @@ __global__ __launch_bounds__(256) void gdr_bwd_mats(GdrArgs a, GdrWs w) {
 template <int DT>
 __global__ __launch_bounds__(256) void gdr_bwd_rows(GdrArgs a, GdrWs w, void *dv) {
     const int64_t ch = blockIdx.x, n = ch / a.H, h = ch % a.H, KP = w.KP, VP = w.VP;
-    const int len = w.chunk_len[n];
+    const int len = w.plan.len(n);
     if (len == 0) return;
-    const int64_t tok0 = w.chunk_tok0[n];
+    const int64_t tok0 = w.plan.tok0(n);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, kt = (int)(KP / 64);
     __shared__ float4 smem[2 * kPanels / 4];
     __shared__ float bet[kChunk], bg[kChunk], red[4][2 * kChunk];
@@ -1020,9 +1009,9 @@ template <int DT>
 __global__ __launch_bounds__(256) void gdr_bwd_finish(GdrArgs a, GdrWs w, void *dq, void *dk, void *dg,
                                                       void *dbeta) {
     const int64_t ch = blockIdx.x, n = ch / a.H, h = ch % a.H, KP = w.KP, VP = w.VP;
-    const int len = w.chunk_len[n];
+    const int len = w.plan.len(n);
     if (len == 0) return;
-    const int64_t tok0 = w.chunk_tok0[n], Dk = a.Dk;
+    const int64_t tok0 = w.plan.tok0(n), Dk = a.Dk;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, kt = (int)(KP / 64), vt = (int)(VP / 64);
     __shared__ float dots[2][kChunk], inv[2][kChunk];
     const float *pt = w.part + ch * w.npart;
@@ -1112,11 +1101,7 @@ size_t gdr_ws_layout(const dm_gdr_desc *d, bool backward, char *base, GdrWs *w) 
         return p;
     };
     auto rows = [&](int64_t a, int64_t b) { return (float *)take((size_t)(ch * a * b) * 4); };
-    x.seq_chunk0 = (int32_t *)take((S + 1) * 4);
-    x.chunk_seq = (int32_t *)take(nc * 4);
-    x.chunk_tok0 = (int32_t *)take(nc * 4);
-    x.chunk_len = (int32_t *)take(nc * 4);
-    x.seq_order = (int32_t *)take(S * 4);
+    x.plan = gdr_plan_layout(d, take);
     x.G = (double *)rows(C, 2);
     x.qn = rows(C, KP);
     x.kn = rows(C, KP);
@@ -1200,17 +1185,11 @@ GdrArgs gdr_args(const dm_gdr_desc *d, const void *q, const void *k, const void 
     return a;
 }
 
-int launch_plan(const dm_gdr_desc *d, int32_t *seq_chunk0, int32_t *chunk_seq,
-                int32_t *chunk_tok0, int32_t *chunk_len, hipStream_t st, int32_t *seq_order) {
-    const int64_t nc = gdr_chunk_bound(d), S = gdr_nseq(d);
-    gdr_plan<<<1, 1024, 0, st>>>(S, d->t, nc, d->cu_seqlens, seq_chunk0, chunk_seq, chunk_tok0,
-                                chunk_len, seq_order);
+int launch_plan(const dm_gdr_desc *d, const GdrPlan &p, hipStream_t st) {
+    if (p.closed) return DM_OK;
+    gdr_plan<<<1, 1024, 0, st>>>(gdr_nseq(d), d->t, gdr_chunk_bound(d), d->cu_seqlens, p);
     DM_LAUNCH_CHECK("chunk_gated_delta_rule: plan");
     return DM_OK;
-}
-
-int launch_gdr_plan(const dm_gdr_desc *d, GdrWs &w, hipStream_t st) {
-    return launch_plan(d, w.seq_chunk0, w.chunk_seq, w.chunk_tok0, w.chunk_len, st, w.seq_order);
 }
 
 template <bool BWD>
@@ -1269,7 +1248,7 @@ int dm_gdr_chunk_fwd(const dm_gdr_desc *d, const void *q, const void *k, const v
     GdrWs w;
     gdr_ws_layout(d, false, (char *)workspace, &w);
     GdrArgs a = gdr_args(d, q, k, v, g, beta);
-    if ((rc = launch_gdr_plan(d, w, st))) return rc;
+    if ((rc = launch_plan(d, w.plan, st))) return rc;
     const unsigned chunks = (unsigned)(nc * d->h);
     const unsigned vt = (unsigned)(w.VP / 64);
 #define FWD(DT)                                                                        \
@@ -1319,7 +1298,7 @@ int dm_gdr_chunk_bwd(const dm_gdr_desc *d, const void *q, const void *k, const v
     GdrWs w;
     gdr_ws_layout(d, true, (char *)workspace, &w);
     GdrArgs a = gdr_args(d, q, k, v, g, beta);
-    if ((rc = launch_gdr_plan(d, w, st))) return rc;
+    if ((rc = launch_plan(d, w.plan, st))) return rc;
     const unsigned chunks = (unsigned)(nc * d->h);
     const unsigned kt = (unsigned)(w.KP / 64), vt = (unsigned)(w.VP / 64);
 #define BWD(DT)                                                                              \

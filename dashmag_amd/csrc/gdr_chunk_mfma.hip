@@ -40,8 +40,7 @@ constexpr int kTrS = kD + 32;   // row stride read by ds_read_b64_tr_b16
 
 struct MfmaWs {
     int64_t nsh;       // sequences x heads
-    int32_t *seq_chunk0, *chunk_seq, *chunk_tok0, *chunk_len;
-    int32_t *seq_order;  // [S]: the sequences by chunk count, the most first
+    GdrPlan plan;
     float *G;          // [ch][64]
     uint16_t *Wf;      // [ch][2 token tiles][8 dk steps][64 lanes][8]: W as A fragments of V' = W S
     uint16_t *Uc;      // [ch][4 dv tiles][2 token tiles][2][64 lanes][8]: U in the product layout
@@ -71,11 +70,7 @@ static size_t mfma_layout(const dm_gdr_desc *d, char *base, MfmaWs *w, bool bwd 
     };
     MfmaWs x{};
     x.nsh = S * d->h;
-    x.seq_chunk0 = (int32_t *)take((S + 1) * 4);
-    x.chunk_seq = (int32_t *)take(nc * 4);
-    x.chunk_tok0 = (int32_t *)take(nc * 4);
-    x.chunk_len = (int32_t *)take(nc * 4);
-    x.seq_order = (int32_t *)take(S * 4);
+    x.plan = gdr_plan_layout(d, take);
     x.G = (float *)take(ch * kC * 4);
     x.Wf = (uint16_t *)take(ch * kC * kD * 2);
     x.Uc = (uint16_t *)take(ch * kC * kD * 2);
@@ -181,9 +176,9 @@ template <int DT>
 __global__ __launch_bounds__(256, 3) void gdr_mfma_prep(GdrArgs a, MfmaWs w) {
     __shared__ PrepSmem sm;
     const int64_t ch = blockIdx.x, n = ch / a.H, h = ch % a.H;
-    const int len = w.chunk_len[n];
+    const int len = w.plan.len(n);
     if (len == 0) return;
-    const int64_t tok0 = w.chunk_tok0[n];
+    const int64_t tok0 = w.plan.tok0(n);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int col = lane & 31, half = lane >> 5;
     uint16_t *ks = (uint16_t *)sm.k, *qs = (uint16_t *)sm.q;
@@ -620,13 +615,13 @@ __global__ __launch_bounds__(256, 3) void gdr_mfma_prep(GdrArgs a, MfmaWs w) {
 // plan's sequence order, the longest chains first, so they are dispatched first. Grid:
 // state_grid(nsh) workgroups.
 __host__ __device__ inline int64_t state_grid(int64_t nsh) { return (nsh + 7) / 8 * 32; }
-__device__ __forceinline__ bool state_item(int64_t x, int64_t nsh, const int32_t *order,
+__device__ __forceinline__ bool state_item(int64_t x, int64_t nsh, const GdrPlan &plan,
                                            int64_t H, int64_t *sh, int *wave) {
     const int64_t xcd = x % 8, y = x / 8;
     *wave = (int)(y % 4);
     const int64_t idx = (y / 4) * 8 + xcd;
     if (idx >= nsh) return false;
-    *sh = (int64_t)order[idx / H] * H + idx % H;
+    *sh = plan.order(idx / H) * H + idx % H;
     return true;
 }
 
@@ -699,8 +694,8 @@ __device__ __forceinline__ void state_output(const GdrArgs &a, const MfmaWs &w, 
     // in the chunk loop waits on another)
     int64_t first = 0, end = 0;
     if (c0 < c1) {
-        first = w.chunk_tok0[c0];
-        end = (int64_t)w.chunk_tok0[c1 - 1] + w.chunk_len[c1 - 1];
+        first = w.plan.tok0(c0);
+        end = (int64_t)w.plan.tok0(c1 - 1) + w.plan.len(c1 - 1);
     }
     // the block's output columns blk * 32 + [0, 32) of the rows
     uint16_t *obase0 = (uint16_t *)out + h * a.Dv + blk * 32;
@@ -798,12 +793,12 @@ __global__ __launch_bounds__(64 * NP + (OUT ? 128 : 0), 1) void gdr_mfma_state2(
     __shared__ __align__(16) uint16_t otiles[OUT ? 2 * 32 * kOutRow : 8];
     int64_t sh;
     int blk;
-    if (!state_item(blockIdx.x, w.nsh, w.seq_order, a.H, &sh, &blk)) return;
+    if (!state_item(blockIdx.x, w.nsh, w.plan, a.H, &sh, &blk)) return;
     const int64_t s = sh / a.H, h = sh % a.H;
     const int lane = threadIdx.x & 63;
     const int p = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // row part (>= NP: output)
     const int col = lane & 31;
-    const int c0 = w.seq_chunk0[s], c1 = w.seq_chunk0[s + 1];
+    const int c0 = w.plan.first(s), c1 = w.plan.first(s + 1);
     const int dv = blk * 32 + col;
     if (OUT && p >= NP) {
 #ifdef DM_TRACE_STATE
@@ -1056,9 +1051,9 @@ template <int DT>
 __global__ __launch_bounds__(256) void gdr_bwd_pre(GdrArgs a, MfmaWs w, const void *d_out) {
     __shared__ BwdPreSmem sm;
     const int64_t ch = blockIdx.x, n = ch / a.H, h = ch % a.H;
-    const int len = w.chunk_len[n];
+    const int len = w.plan.len(n);
     if (len == 0) return;
-    const int64_t tok0 = w.chunk_tok0[n];
+    const int64_t tok0 = w.plan.tok0(n);
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint16_t *dob = (const uint16_t *)d_out, *qin = (const uint16_t *)a.q;
@@ -1156,12 +1151,12 @@ __global__ __launch_bounds__(128, 1) void gdr_bwd_state2(GdrArgs a, MfmaWs w, co
     __shared__ __align__(16) float4 xch[2][2][2][4][64];  // [parity][wavefront][token tile][i / 4][lane]
     int64_t sh;
     int blk;
-    if (!state_item(blockIdx.x, w.nsh, w.seq_order, a.H, &sh, &blk)) return;
+    if (!state_item(blockIdx.x, w.nsh, w.plan, a.H, &sh, &blk)) return;
     const int64_t s = sh / a.H, h = sh % a.H;
     const int lane = threadIdx.x & 63;
     const int p = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // row half
     const int col = lane & 31;
-    const int c0 = w.seq_chunk0[s], c1 = w.seq_chunk0[s + 1];
+    const int c0 = w.plan.first(s), c1 = w.plan.first(s + 1);
     const int dv = blk * 32 + col;
     // dS_p: tile r holds rows 64 p + 32 r + crow(i) of column dv
     f32x16_t D[2];
@@ -1369,9 +1364,9 @@ __global__ __launch_bounds__(512, 1) void gdr_bwd_grads(GdrArgs a, MfmaWs w, con
                                                         void *dbeta) {
     __shared__ __align__(16) char smem[bl::BYTES];
     const int64_t ch = blockIdx.x, n = ch / a.H, h = ch % a.H;
-    const int len = w.chunk_len[n];
+    const int len = w.plan.len(n);
     if (len == 0) return;
-    const int64_t tok0 = w.chunk_tok0[n];
+    const int64_t tok0 = w.plan.tok0(n);
     const int tid = threadIdx.x, lane = tid & 63;
     DM_GSTAMP(0);
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1964,7 +1959,7 @@ int launch_gdr_mfma_fwd(const dm_gdr_desc *d, const void *q, const void *k, cons
     mfma_layout(d, (char *)workspace, &w);
     const GdrArgs a = gdr_args(d, q, k, v, g, beta);
     const int64_t nc = gdr_chunk_bound(d), S = gdr_nseq(d);
-    int rc = launch_plan(d, w.seq_chunk0, w.chunk_seq, w.chunk_tok0, w.chunk_len, st, w.seq_order);
+    int rc = launch_plan(d, w.plan, st);
     if (rc) return rc;
     const unsigned chunks = (unsigned)(nc * d->h), seqs = (unsigned)(S * d->h);
     if (d->dtype == DM_BF16) {
@@ -2034,7 +2029,7 @@ int launch_gdr_mfma_bwd(const dm_gdr_desc *d, const void *q, const void *k, cons
     mfma_layout(d, (char *)workspace, &w, true);
     const GdrArgs a = gdr_args(d, q, k, v, g, beta);
     const int64_t nc = gdr_chunk_bound(d), S = gdr_nseq(d);
-    int rc = launch_plan(d, w.seq_chunk0, w.chunk_seq, w.chunk_tok0, w.chunk_len, st, w.seq_order);
+    int rc = launch_plan(d, w.plan, st);
     if (rc) return rc;
     const unsigned chunks = (unsigned)(nc * d->h), seqs = (unsigned)(S * d->h);
     if (d->dtype == DM_BF16)

@@ -43,11 +43,28 @@ __host__ __device__ inline int64_t o_at(const GdrArgs &a, int64_t tok, int64_t h
 bool gdr_strides_ok(const dm_gdr_desc *d, bool step);
 bool gdr_strides_16b(const dm_gdr_desc *d);
 
+// Which tokens each chunk holds and which chunks each sequence: the arrays gdr_plan writes for
+// packed sequences, or, for a batch of sequences of T tokens, in closed form from its `per` chunks a
+// sequence (a launch and its latency less: 6144 tokens forward 143 -> 137 us).
+struct GdrPlan {
+    int32_t *seq_chunk0, *chunk_tok0, *chunk_len;  // [S + 1], [chunks], [chunks]
+    int32_t *seq_order;                            // [S]: the sequences by chunk count, the most first
+    int32_t closed, T, per;                        // closed: no arrays
+    __device__ __forceinline__ int len(int64_t n) const {
+        return closed ? min(kChunk, T - (int32_t)n % per * kChunk) : chunk_len[n];
+    }
+    __device__ __forceinline__ int64_t tok0(int64_t n) const {
+        return closed ? (int64_t)((int32_t)n / per) * T + (int32_t)n % per * kChunk : chunk_tok0[n];
+    }
+    __device__ __forceinline__ int first(int64_t s) const { return closed ? (int32_t)s * per : seq_chunk0[s]; }
+    __device__ __forceinline__ int64_t order(int64_t i) const { return closed ? i : seq_order[i]; }
+};
+
 // The f32 kernels' workspace: the plan, then per (chunk, head) f32 intermediates, rows of KP and
 // VP columns (Dk and Dv padded with zeros to multiples of 64); names ending in T are transposed.
 struct GdrWs {
     int64_t KP, VP, npart;
-    int32_t *seq_chunk0, *chunk_seq, *chunk_tok0, *chunk_len, *seq_order;
+    GdrPlan plan;
     double *G;  // cumulative log-decay
     float *qn, *kn, *vp, *P, *W, *KT, *UT, *ScT, *VnT;
     // the backward's
@@ -55,15 +72,28 @@ struct GdrWs {
 };
 
 int check_gdr(const dm_gdr_desc *d, const char *op, bool step);
-// The chunk plan over the call's sequences (gdr_chunk.hip).
-// seq_order (optional, [nseq]): the sequences by chunk count, the most first (ties by index),
-// for at most kOrderMax sequences; the identity beyond.
+// The longest-first order is kept for at most kOrderMax sequences; the identity beyond.
 constexpr int64_t kOrderMax = 4096;
-int launch_plan(const dm_gdr_desc *d, int32_t *seq_chunk0, int32_t *chunk_seq,
-                int32_t *chunk_tok0, int32_t *chunk_len, hipStream_t st,
-                int32_t *seq_order = nullptr);
 int64_t gdr_nseq(const dm_gdr_desc *d);
 int64_t gdr_chunk_bound(const dm_gdr_desc *d);
+// The plan's place in a workspace, and its launch (gdr_chunk.hip).
+template <class F>
+GdrPlan gdr_plan_layout(const dm_gdr_desc *d, F take) {
+    const int64_t nc = gdr_chunk_bound(d), S = gdr_nseq(d);
+    GdrPlan p{};
+    if (!d->cu_seqlens) {
+        p.closed = 1;
+        p.T = (int32_t)d->t;
+        p.per = (int32_t)((d->t + kChunk - 1) / kChunk);
+        return p;
+    }
+    p.seq_chunk0 = (int32_t *)take((S + 1) * 4);
+    p.chunk_tok0 = (int32_t *)take(nc * 4);
+    p.chunk_len = (int32_t *)take(nc * 4);
+    p.seq_order = (int32_t *)take(S * 4);
+    return p;
+}
+int launch_plan(const dm_gdr_desc *d, const GdrPlan &p, hipStream_t st);
 
 // MFMA forward and backward (gdr_chunk_mfma.hip): bf16/f16, Dk and Dv multiples of 8 up to 128
 // (the products are 128 wide; columns past a width are held at zero).

@@ -845,7 +845,7 @@ int dm_linear_cross_entropy_bwd(const dm_lce_desc *d, const void *hidden, const 
     // written once, in its own dtype (bf16 with at most one group of rows): accumulated per row
     // block in f32 over the whole vocabulary, 4096 rows of 4096 by 151936 tokens moved 10 GB more
     // (of which 3.7 GB, 720 us, rounded the sum), and its products of 2048 rows each took 165 us a
-    // chunk where one of 4096 takes 240. With more groups an f32 chunk accumulates.
+    // chunk where one of 4096 takes 250. With more groups an f32 chunk accumulates.
     // The first product of each accumulator runs with beta = 0, which hipBLASLt takes as "C is not
     // read" (the accumulators are never cleared; a workspace poisoned with NaN gives the same bits
     // as a zeroed one, a property the GPU tests hold it to).

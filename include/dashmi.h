@@ -251,7 +251,9 @@ int dm_attention_row_bounds(const dm_attention_desc *desc, int64_t b, int64_t i,
                             int64_t *hi);
 
 /* Attention forward: o [B, Tq, Hq, D] in dtype, lse [B, Tq, Hq] f32 (natural log, -inf for a
- * query that sees no key, whose output is 0). Replaces attention.rs:660 / cube.rs:562. */
+ * query that sees no key, whose output is 0). The workspace may be NULL: a call of few queries,
+ * which the query asks one for to split the keys over more workgroups, then runs in one piece.
+ * Replaces attention.rs:660 / cube.rs:562. */
 size_t dm_attention_fwd_workspace(const dm_attention_desc *desc);
 int dm_attention_fwd(const dm_attention_desc *desc, const void *q, const void *k, const void *v,
                      void *o, float *lse, void *workspace, size_t workspace_bytes, void *stream);
@@ -400,8 +402,8 @@ int dm_chosen_logprob(const dm_logprob_desc *desc, const void *hidden, const voi
  * LinearCrossEntropyBackend::linear_cross_entropy (loss.rs:134-160; the written-out backward is
  * always taken, as with a weight that trains). The workspace query's `backward`: 0 for the
  * forward, 1 for a backward with both gradients, 2 for a backward without grad_weight (a frozen
- * output weight: no V x D f32 accumulator is reserved; the backward then refuses a non-NULL
- * grad_weight with that smaller workspace). */
+ * output weight: no f32 accumulator for a chunk of it is reserved; the backward then refuses a
+ * non-NULL grad_weight with that smaller workspace). */
 size_t dm_linear_cross_entropy_workspace(const dm_lce_desc *desc, int backward);
 int dm_linear_cross_entropy_fwd(const dm_lce_desc *desc, const void *hidden, const void *weight,
                                 const int64_t *targets, const uint32_t *masked, int64_t n_masked,

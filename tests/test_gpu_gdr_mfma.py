@@ -123,3 +123,32 @@ def test_mfma_backward_matches_oracle(dtype, lens, h, l2norm, tol, states):
         worst = max(worst, rr)
         print(f"  {name}: rel {rr:.2e}")
     assert worst <= tol
+
+
+@pytest.mark.parametrize("B,T,dtype", [
+    (3, 100, torch.bfloat16), (2, 64, torch.float16), (5, 1, torch.bfloat16),
+    (2, 130, torch.float32),
+])
+def test_batch_without_offsets_equals_packed(B, T, dtype):
+    """Sequences of one length without offsets (their chunks known in closed form) and the same
+    ones packed with offsets (their chunks from a table): the same arithmetic, to the bit."""
+    H, D = 3, 128
+    seed = 900 + B + T
+    q, k, v, do = (syn.normal(seed + i, (B, T, H, D), "cuda").to(dtype) for i in range(4))
+    g = -torch.nn.functional.softplus(syn.normal(seed + 4, (B, T, H), "cuda"))
+    beta = torch.sigmoid(syn.normal(seed + 5, (B, T, H), "cuda"))
+    st = syn.normal(seed + 6, (B, H, D, D), "cuda", std=0.1)
+    cu = torch.arange(0, (B + 1) * T, T, dtype=torch.int32).cuda()
+    opts = dm.ChunkGatedDeltaOptions(qk_l2norm=True, output_final_state=True)
+    print(f"case {B} x {T} {dtype}", flush=True)
+
+    def run(pack):
+        f = (lambda x: x.reshape(1, B * T, *x.shape[2:])) if pack else (lambda x: x)
+        a = [f(x) for x in (q, k, v, g, beta)] + [st, cu if pack else None]
+        got = list(dm.chunk_gated_delta_rule(*a, opts))
+        got += dm.chunk_gated_delta_rule_backward(*a, f(do), st, opts)
+        torch.cuda.synchronize()
+        return got
+
+    for i, (x, y) in enumerate(zip(run(False), run(True))):
+        assert torch.equal(x.reshape(y.shape), y), i

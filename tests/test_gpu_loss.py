@@ -6,7 +6,8 @@ the coefficients and the logits' gradient), against the reference's PyTorch-floa
 relative to max|want|: f32 [2e-7, 2e-7, 1e-6, 4e-6, 4e-6]; bf16 [2e-7, 2e-7, 3e-7, 5e-3, 5e-3]
 (the logits' gradient rounded to bf16 for the products, the gradients returned in bf16). Also:
 each term's gradient alone, chunking, f16 inputs against f32 inputs of the same values
-(loss.rs:934: [2e-7, 2e-7, 1e-6, 1e-3, 1e-3]), an empty batch, every row ignored, agreement with
+(loss.rs:934: [2e-7, 2e-7, 1e-6, 1e-3, 1e-3]), several groups of
+rows, an empty batch, every row ignored, agreement with
 the chosen-token log-probability, the refusals."""
 import numpy as np
 import pytest
@@ -80,6 +81,41 @@ def test_chunking_does_not_change_the_answer(chunks):
     print(f"loss peaked smooth f32 {chunks}", flush=True)
     c = Case("peaked")
     _check(_run(c, "f32", "smooth", chunks=chunks), c.want("f32", "smooth"), BOUNDS["f32"])
+
+
+@pytest.mark.parametrize("dtype,n,d,chunks", [
+    ("bf16", 20000, 64, dict(vocab_chunk=128, row_chunk=3072)),  # two groups of rows
+    ("f16", 20000, 64, dict(vocab_chunk=128, row_chunk=3072)),
+    ("f32", 20000, 64, dict(vocab_chunk=128, row_chunk=3072)),
+    ("f32", 16385, 24, dict(vocab_chunk=0, row_chunk=1)),  # the second group of one row
+    ("bf16", 70, 8, dict(vocab_chunk=7, row_chunk=33)),  # rows of the logits' gradient of 14 bytes
+])
+def test_row_groups_and_odd_chunks(dtype, n, d, chunks):
+    """The gradients against float64, where the weight's is summed over several groups of rows in
+    an f32 chunk, or over chunks of an odd width. Bounds, of the largest value: f32 the
+    recorded cases' 4e-6 and a sum over n rows in f32, sqrt(n) 2^-24 (both directions of rounding
+    equally likely); f16 and bf16 the bounds above, 1e-3 and 5e-3 (the sum's own is below them),
+    f16's with 2^-25 / max|want|: the mean over 20000 rows leaves grad_hidden below f16's normal
+    range (2^-14), where a rounding is up to 2^-25 whatever the value."""
+    print(f"loss {dtype} n {n} d {d} {chunks}", flush=True)
+    v, gen = 300, torch.Generator().manual_seed(n + d)
+    h = torch.randn(n, d, generator=gen).to(DT[dtype])
+    w = (torch.randn(v, d, generator=gen) * d ** -0.5).to(DT[dtype])
+    t = torch.randint(0, v, (n,), generator=gen)
+    opts = dm.CrossEntropyOptions(chunks=dm.LogprobOptions(**chunks))
+    hd, wd = h.cuda(), w.cuda()
+    rows = dm.linear_cross_entropy(hd, wd, t, opts)[3]
+    up = torch.stack([torch.full((n,), 1.0 / n), torch.zeros(n), torch.zeros(n)])
+    got = dm.linear_cross_entropy_backward(hd, wd, t, rows, up, opts)
+    torch.cuda.synchronize()
+    h64, w64 = h.double().requires_grad_(), w.double().requires_grad_()
+    torch.nn.functional.cross_entropy(h64 @ w64.T, t).backward()
+    bound = {"f32": 4e-6 + n ** 0.5 * 2 ** -24, "f16": 1e-3, "bf16": 5e-3}[dtype]
+    for part, g, e in zip(PARTS[3:], got, (h64.grad, w64.grad)):
+        r = rel_error(g.float().cpu().numpy(), e.numpy())
+        b = bound + (2 ** -25 / float(e.abs().max()) if dtype == "f16" else 0)
+        print(f"{part}: {r:.2e} (bound {b:.1e})")
+        assert r <= b, (part, r, b)
 
 
 @pytest.mark.parametrize("name", CASES)

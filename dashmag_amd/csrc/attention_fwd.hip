@@ -31,10 +31,14 @@ namespace dm {
 template <int D>
 constexpr int fwd_waves() { return D == 256 ? 4 : 8; }
 // Wavefronts a SIMD the registers are held to. At width 64 128 registers (of 140 taken freely)
-// let two workgroups share a compute unit: unmasked 6144 queries and keys of 32 heads 420 -> 365 us,
-// of 128 heads 1470 -> 1264 us (841 -> 979 TFLOP/s).
-template <int D>
-constexpr int fwd_simd_waves() { return D == 64 ? 4 : 1; }
+// let two workgroups share a compute unit (PAIR): unmasked 6144 queries and keys of 32 heads 361 -> 329
+// us, causal of 64 heads 395 -> 343. Taken by calls of kPairItems work items or more, and of more than
+// one a compute unit where all are of one length (no causal mask, window or packing): with fewer, two
+// of the longest share a unit and end the call late (2 x 3072 causal of 16 heads, 384 items, 65 us
+// alone and 80 paired, of 24 heads 101 and 102, of 32 heads, 768 items, 120 and 102).
+template <int D, bool PAIR>
+constexpr int fwd_simd_waves() { return D == 64 && PAIR ? 4 : 1; }
+constexpr int64_t kPairItems = 768;
 constexpr int kFwdN = 64;   // keys per tile
 
 // Row strides (elements) of the LDS tiles: K rows are read along D by ds_read_b128 (16 lanes on
@@ -97,8 +101,8 @@ __device__ __forceinline__ int split_tile(const FwdSplit &sp, int ntiles, int c)
     return lo;
 }
 
-template <int DT, int D, bool PAD, bool SPLIT>
-__global__ __launch_bounds__(64 * fwd_waves<D>(), fwd_simd_waves<D>()) void attn_fwd_mfma(MaskInfo m, int64_t B, int64_t Hq,
+template <int DT, int D, bool PAD, bool SPLIT, bool PAIR>
+__global__ __launch_bounds__(64 * fwd_waves<D>(), (fwd_simd_waves<D, PAIR>())) void attn_fwd_mfma(MaskInfo m, int64_t B, int64_t Hq,
                                                       int64_t Hkv, float scale, AttnStrides sd,
                                                       const uint16_t *__restrict__ q,
                                                       const uint16_t *__restrict__ k,
@@ -475,7 +479,7 @@ extern "C" int dm_debug_trace_fwd(void *host, size_t bytes) {
 // is 36. Of the segment lengths that cut the longest item in up to 16, the one is taken whose
 // workgroups, laid on 256 compute units longest first, end earliest, each workgroup costing
 // kSegCost tiles besides its own (its start, its partial outputs) and the split kMergeCost (the
-// merge). Measured, before and after: 6144 causal queries of 8 heads, width 64: 125 -> 75 us; width 128, 2048
+// merge). Measured, before and after: 6144 causal queries of 8 heads, width 64: 117 -> 75 us; width 128, 2048
 // queries: 58 -> 35, 4096: 108 -> 65, 6144: 155 -> 110; width 256, 2048: 92 -> 56; 16 queries against 8192
 // keys of 8 heads of 128: 152 -> 28; unmasked 6144 of width 64 (192 equal items) are as fast whole.
 static size_t fwd_split(const dm_attention_desc *d, char *base, FwdSplit *sp) {
@@ -484,17 +488,25 @@ static size_t fwd_split(const dm_attention_desc *d, char *base, FwdSplit *sp) {
     const int64_t nt = (d->tq + per - 1) / per, rows = d->hq * d->b;
     sp->nseg = 0;
     if (nt * rows == 0 || nt * rows >= kCUs || d->tk <= kMinTiles * kFwdN) return 0;
-    // key tiles of each query tile, from the mask's closed form (offsets lie on the device: packed
-    // sequences are taken for one)
+    if (d->mask_kind == DM_MASK_PACKED && d->nseq > 2) return 0;
+    // Key tiles of each query tile, from the mask's closed form. Offsets lie on the device: two packed
+    // sequences are taken for equal ones, and calls of more run whole (equal lengths taken for one
+    // sequence, 4 x 1536 causal tokens of 8 heads of 64, took 54 us against 36 whole; 5000, 500, 400 and
+    // 244 taken for equal ones 143 against 131).
     MaskInfo m = mask_info(d);
+    const int64_t ns = m.kind == DM_MASK_PACKED ? std::max<int64_t>(d->nseq, 1) : 1;
     m.kind = DM_MASK_NONE;
+    m.tq = (d->tq + ns - 1) / ns;
+    m.tk = (d->tk + ns - 1) / ns;
     const int ntiles = (int)nt;
     int n[kSplitTiles], most = 0;
     for (int t = 0; t < ntiles; t++) {
         int64_t lo, hi, x;
-        const int64_t q0 = (ntiles - 1 - t) * per;
-        row_bounds(m, q0, &lo, &x);
-        row_bounds(m, std::min(q0 + per, d->tq) - 1, &x, &hi);
+        const int64_t q0 = (ntiles - 1 - t) * per, q1 = std::min(q0 + per, d->tq) - 1;
+        row_bounds(m, q0 % m.tq, &lo, &x);
+        row_bounds(m, q1 % m.tq, &x, &hi);
+        lo += q0 / m.tq * m.tk;
+        hi += q1 / m.tq * m.tk;
         n[t] = (int)std::max<int64_t>((hi - lo + kFwdN - 1) / kFwdN, 1);
         most = std::max(most, n[t]);
     }
@@ -568,13 +580,17 @@ int launch_attn_fwd_mfma(const MaskInfo &m, const dm_attention_desc *d, float sc
     const uint16_t *qq = (const uint16_t *)q, *kk = (const uint16_t *)k, *vv = (const uint16_t *)v;
     uint16_t *oo = (uint16_t *)o;
     const AttnStrides sd = attn_strides(d);
+    const bool equal = m.right < 0 && m.left < 0 && m.kind != DM_MASK_PACKED;
+    const bool pair = d->d == 64 && (split || nwork >= kPairItems || (equal && nwork > 256));
 #define FWD1(DT, DD, PAD, SPLIT)                                                                  \
-    attn_fwd_mfma<DT, DD, PAD, SPLIT><<<grid, block, 0, st>>>(m, d->b, d->hq, d->hkv, scale, sd, qq, \
+    if (pair) FWD2(DT, DD, PAD, SPLIT, DD == 64); else FWD2(DT, DD, PAD, SPLIT, DD == 64 && SPLIT)
+#define FWD2(DT, DD, PAD, SPLIT, PAIR)                                                            \
+    attn_fwd_mfma<DT, DD, PAD, SPLIT, PAIR><<<grid, block, 0, st>>>(m, d->b, d->hq, d->hkv, scale, sd, qq, \
                                                               kk, vv, oo, lse, sp)
 #define FWD(DT, DD)                                                                                   \
     {                                                                                                 \
         if (split) {                                                                                  \
-            if (m.pad) FWD1(DT, DD, true, true); else FWD1(DT, DD, false, true);                      \
+            if (m.pad) { FWD1(DT, DD, true, true); } else { FWD1(DT, DD, false, true); }              \
             attn_fwd_merge<DT, DD><<<dim3((unsigned)nwork, (unsigned)(per * DD / 1024)), 256, 0, st>>>( \
                 d->tq, d->hq, d->hkv, d->b, (int)ntiles, sp, oo, lse);                                           \
         } else if (m.pad) {                                                                           \
@@ -593,6 +609,7 @@ int launch_attn_fwd_mfma(const MaskInfo &m, const dm_attention_desc *d, float sc
     }
 #undef FWD
 #undef FWD1
+#undef FWD2
     probe_add(DM_PROBE_ATTN_FWD_MFMA);
     DM_LAUNCH_CHECK("attention: MFMA forward launch");
     return DM_OK;

@@ -26,7 +26,7 @@ CASES = [
     ("causal_empty_rows_1800x1500", 1, 1800, 1500, 2, 2, None, True, None, None),
     ("window_1800", 1, 1800, 1800, 2, 1, None, True, (1000, U), None),
     ("padding_1700_b3", 3, 1700, 1700, 1, 1, "padding", False, None, None),
-    ("packed_1700", 1, None, None, 2, 1, ("packed", [1500, 0, 200], [1500, 0, 200], 30), True, None,
+    ("packed_3200", 1, None, None, 2, 1, ("packed", [3000, 200], [3000, 200], 30), True, None,
      None),
 ]
 

@@ -88,6 +88,75 @@ __device__ __forceinline__ f32x4_t rows_dot(const float4 (&a)[NS], const float4 
     return (x[0] + x[1]) + (x[2] + x[3]);
 }
 
+// What a row does not see must not reach it, whatever it holds (the positions past the last packed
+// sequence, a later token), and a product's zero weight does not see to that: 0 * inf is NaN. So of a
+// tile of 16 x 16 pairs the terms that no row sees are cleared, as padded ones; and where some rows see a
+// term and others don't, values that are not finite are cleared too, and a wavefront that met one goes
+// over its tiles again after the loop and adds them to the rows that see them (in the loop that code
+// would take the registers of the next tile's loads: 724 bytes a lane spilled at width 256). Tiles of
+// seen pairs alone branch past all of it. 1024 causal tokens of 8 heads, forward and backward, without
+// any of this and with it: width 64 168 and 167 us, 128 270 and 288, 256 581 and 587.
+struct Hidden {
+    bool seen[4];  // lane (c, g): whether any row sees term 4 g + r
+    bool cut;      // some row (of those that are kept) does not see a term that another sees
+    __device__ __forceinline__ Hidden(const bool (&on)[4], bool kept) {
+        const int g = (threadIdx.x >> 4) & 3;
+        bool part = false;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            seen[r] = ((__ballot(on[r]) >> (16 * g)) & 0xffff) != 0;
+            part |= kept && seen[r] && !on[r];
+        }
+        cut = __any(part);
+    }
+    // Whether values were cleared that some row sees.
+    template <int N>
+    __device__ __forceinline__ bool clear(f32x4_t (&x)[N]) const {
+#pragma unroll
+        for (int s = 0; s < N; s++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) x[s][r] = seen[r] ? x[s][r] : 0.f;
+        if (!cut) return false;
+        bool bad = false;
+#pragma unroll
+        for (int s = 0; s < N; s++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const bool fin = fabsf(x[s][r]) < INFINITY;
+                bad |= !fin;
+                x[s][r] = fin ? x[s][r] : 0.f;
+            }
+        return __any(bad);
+    }
+};
+// No pair of the tile is hidden: the terms are taken as they are.
+__device__ __forceinline__ bool all_seen(const bool (&on)[4]) { return __all(on[0] && on[1] && on[2] && on[3]); }
+// x . y over D elements, in the four lanes (c, 0 .. 3) of a row.
+template <int DT>
+__device__ __forceinline__ float dot4(const void *x, int64_t xo, const void *y, int64_t yo, int D) {
+    float t = 0.f;
+    for (int d = (threadIdx.x >> 4) & 3; d < D; d += 4) t += ld<DT>(x, xo + d) * ld<DT>(y, yo + d);
+    t += __shfl_xor(t, 16, 64);
+    return t + __shfl_xor(t, 32, 64);
+}
+// acc[s][e] += w * (element 16 s + 4 g + e at `off`) over the elements that are not finite, where the
+// lane's row sees them.
+template <int DT, int NS>
+__device__ __forceinline__ void add_not_finite(f32x4_t (&acc)[NS], const void *p, int64_t off, bool see, float w,
+                                               int D) {
+    const int g = (threadIdx.x >> 4) & 3;
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int d = 16 * s + 4 * g + e;
+            const float v = see && d < D ? ld<DT>(p, off + d) : 0.f;
+            acc[s][e] = fabsf(v) < INFINITY ? acc[s][e] : fmaf(w, v, acc[s][e]);
+        }
+        __builtin_amdgcn_sched_barrier(0);  // (all the loads at once would take the registers)
+    }
+}
+
 // The smallest lo and largest hi of a tile's rows (lane c's row in lanes c, c + 16, ...); [0, 0)
 // where none sees a key.
 __device__ __forceinline__ int2 tile_union(int lo, int hi) {
@@ -105,8 +174,9 @@ __device__ __forceinline__ float across4(float x) {  // the four 16-lane groups'
     return x + __shfl_xor(x, 32, 64);
 }
 
+// (at width 64 held to 128 registers, of 136 taken freely: four workgroups a compute unit)
 template <int DT, int DP, bool VEC>
-__global__ __launch_bounds__(64 * kNW) void attn_fwd_f32(AttnF32 a, void *o, float *lse) {
+__global__ __launch_bounds__(64 * kNW, DP == 64 ? 4 : 1) void attn_fwd_f32(AttnF32 a, void *o, float *lse) {
     constexpr int NS = DP / 16, OS = DP + 4;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, g = lane >> 4;
     const int D = (int)a.D;
@@ -122,30 +192,32 @@ __global__ __launch_bounds__(64 * kNW) void attn_fwd_f32(AttnF32 a, void *o, flo
     if (i < Tq) row_bounds(a.m, i, &lo, &hi);
     const int2 u = tile_union((int)lo, (int)hi);
     float4 qf[NS], kf[NS];
-    row_load<DT, VEC>(qf, a.q, b * a.sd.q.b + (i < Tq ? i : Tq - 1) * a.sd.q.t + h * a.sd.q.h, D, g);
+    const int64_t qo = b * a.sd.q.b + (i < Tq ? i : Tq - 1) * a.sd.q.t + h * a.sd.q.h;
+    row_load<DT, VEC>(qf, a.q, qo, D, g);
     const int64_t kb = b * a.sd.k.b + kh * a.sd.k.h, vb = b * a.sd.v.b + kh * a.sd.v.h;
     const uint8_t *pad = a.m.pad ? a.m.pad + b * Tk : nullptr;
     // rows past the union are not read: the last row it holds stands in, and is masked
     auto key = [&](int j) { return j < u.y ? j : u.y - 1; };
+    auto sees = [&](int j) { return !(pad && pad[key(j)]) && j >= lo && j < hi; };
     f32x4_t acc[NS];
 #pragma unroll
     for (int s = 0; s < NS; s++) acc[s] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     float mx = -INFINITY, l = 0.f;
+    bool bad = false;
     int j0 = u.x + wave * kQT;
     if (j0 < u.y) row_load<DT, VEC>(kf, a.k, kb + (int64_t)key(j0 + c) * a.sd.k.t, D, g);
     for (; j0 < u.y; j0 += kNW * kQT) {
         int64_t vo[4];
-        bool on[4], drop[4];
+        bool on[4];
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-            const int j = key(j0 + 4 * g + r);
-            vo[r] = vb + (int64_t)j * a.sd.v.t;
-            drop[r] = pad && pad[j];
-            on[r] = !drop[r] && j0 + 4 * g + r >= lo && j0 + 4 * g + r < hi;
+            vo[r] = vb + (int64_t)key(j0 + 4 * g + r) * a.sd.v.t;
+            on[r] = sees(j0 + 4 * g + r);
         }
         f32x4_t vf[NS];
 #pragma unroll
         for (int s = 0; s < NS; s++) vf[s] = col_load<DT>(a.v, vo, 16 * s + c, D);
+        if (!all_seen(on)) bad |= Hidden(on, i < Tq).clear(vf);
         const f32x4_t sv = rows_dot(kf, qf);
         if (j0 + kNW * kQT < u.y)
             row_load<DT, VEC>(kf, a.k, kb + (int64_t)key(j0 + kNW * kQT + c) * a.sd.k.t, D, g);
@@ -173,8 +245,21 @@ __global__ __launch_bounds__(64 * kNW) void attn_fwd_f32(AttnF32 a, void *o, flo
 #pragma unroll
         for (int s = 0; s < NS; s++)
 #pragma unroll
-            for (int r = 0; r < 4; r++)
-                acc[s] = mfma4(drop[r] ? 0.f : vf[s][r], p[r], acc[s]);  // a padded row may hold anything
+            for (int r = 0; r < 4; r++) acc[s] = mfma4(vf[s][r], p[r], acc[s]);
+    }
+    if (bad) {
+        const float ref = mx == -INFINITY ? 0.f : mx;
+        for (j0 = u.x + wave * kQT; j0 < u.y; j0 += kNW * kQT) {
+            const int j = j0 + 4 * g;
+            const bool on[4] = {sees(j), sees(j + 1), sees(j + 2), sees(j + 3)};
+            if (!Hidden(on, i < Tq).cut) continue;
+#pragma unroll 1
+            for (int x = j0; x < j0 + kQT; x++) {
+                const int64_t jx = key(x);
+                const float sc = dot4<DT>(a.q, qo, a.k, kb + jx * a.sd.k.t, D);
+                add_not_finite<DT>(acc, a.v, vb + jx * a.sd.v.t, sees(x), expf(sc * a.scale - ref), D);
+            }
+        }
     }
     l = across4(l);
     if (g == 0) {
@@ -231,8 +316,9 @@ __global__ __launch_bounds__(64 * kNW) void attn_dq_f32(AttnF32 a, void *dq) {
     int2 u = tile_union((int)lo, (int)hi);
     if (h == 0 && threadIdx.x == 0) a.tile[b * nt + qt] = u;
     float4 qf[NS], gf[NS], kf[NS], vf[NS];
-    row_load<DT, VEC>(qf, a.q, b * a.sd.q.b + ic * a.sd.q.t + h * a.sd.q.h, D, g);
-    row_load<DT, VEC>(gf, a.d_o, b * a.sd.g.b + ic * a.sd.g.t + h * a.sd.g.h, D, g);
+    const int64_t qo = b * a.sd.q.b + ic * a.sd.q.t + h * a.sd.q.h, go = b * a.sd.g.b + ic * a.sd.g.t + h * a.sd.g.h;
+    row_load<DT, VEC>(qf, a.q, qo, D, g);
+    row_load<DT, VEC>(gf, a.d_o, go, D, g);
     row_load<DT, VEC>(kf, a.o, b * a.sd.o.b + ic * a.sd.o.t + h * a.sd.o.h, D, g);
     const int64_t row = (b * Tq + ic) * a.Hq + h;
     const float ls = a.lse[row];
@@ -249,6 +335,9 @@ __global__ __launch_bounds__(64 * kNW) void attn_dq_f32(AttnF32 a, void *dq) {
     const int64_t kb = b * a.sd.k.b + kh * a.sd.k.h, vb = b * a.sd.v.b + kh * a.sd.v.h;
     const uint8_t *pad = a.m.pad ? a.m.pad + b * Tk : nullptr;
     auto key = [&](int j) { return (int64_t)(j < u.y ? j : u.y - 1); };
+    auto sees = [&](int j) { return !(pad && pad[key(j)]) && j >= lo && j < hi; };
+    auto grad = [&](float s, float dp) { return expf(s * a.scale - ls) * (dp - delta); };
+    bool bad = false;
     f32x4_t acc[NS];
 #pragma unroll
     for (int s = 0; s < NS; s++) acc[s] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -260,26 +349,38 @@ __global__ __launch_bounds__(64 * kNW) void attn_dq_f32(AttnF32 a, void *dq) {
     if (j0 < u.y) load(j0);
     for (; j0 < u.y; j0 += kNW * kQT) {
         int64_t ko[4];
-        bool on[4], drop[4];
+        bool on[4];
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-            const int64_t j = key(j0 + 4 * g + r);
-            ko[r] = kb + j * a.sd.k.t;
-            drop[r] = pad && pad[j];
-            on[r] = !drop[r] && j0 + 4 * g + r >= lo && j0 + 4 * g + r < hi;
+            ko[r] = kb + key(j0 + 4 * g + r) * a.sd.k.t;
+            on[r] = sees(j0 + 4 * g + r);
         }
         f32x4_t kc[NS];
 #pragma unroll
         for (int s = 0; s < NS; s++) kc[s] = col_load<DT>(a.k, ko, 16 * s + c, D);
+        if (!all_seen(on)) bad |= Hidden(on, i < Tq).clear(kc);
         const f32x4_t sv = rows_dot(kf, qf), dp = rows_dot(vf, gf);
         if (j0 + kNW * kQT < u.y) load(j0 + kNW * kQT);
         float ds[4];
 #pragma unroll
-        for (int r = 0; r < 4; r++) ds[r] = on[r] ? expf(sv[r] * a.scale - ls) * (dp[r] - delta) : 0.f;
+        for (int r = 0; r < 4; r++) ds[r] = on[r] ? grad(sv[r], dp[r]) : 0.f;
 #pragma unroll
         for (int s = 0; s < NS; s++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) acc[s] = mfma4(drop[r] ? 0.f : kc[s][r], ds[r], acc[s]);
+            for (int r = 0; r < 4; r++) acc[s] = mfma4(kc[s][r], ds[r], acc[s]);
+    }
+    if (bad) {
+        for (j0 = u.x + wave * kQT; j0 < u.y; j0 += kNW * kQT) {
+            const int j = j0 + 4 * g;
+            const bool on[4] = {sees(j), sees(j + 1), sees(j + 2), sees(j + 3)};
+            if (!Hidden(on, i < Tq).cut) continue;
+#pragma unroll 1
+            for (int x = j0; x < j0 + kQT; x++) {
+                const int64_t k0 = kb + key(x) * a.sd.k.t, v0 = vb + key(x) * a.sd.v.t;
+                const float w = grad(dot4<DT>(a.q, qo, a.k, k0, D), dot4<DT>(a.d_o, go, a.v, v0, D));
+                add_not_finite<DT>(acc, a.k, k0, sees(x), w, D);
+            }
+        }
     }
 #pragma unroll
     for (int s = 0; s < NS; s++)
@@ -331,8 +432,9 @@ __global__ __launch_bounds__(64 * kNW) void attn_dkdv_f32(AttnF32 a, void *dk, v
         }
     }
     float4 kf[NS], vf[NS], qf[NS], gf[NS];
-    row_load<DT, VEC>(kf, a.k, b * a.sd.k.b + jc * a.sd.k.t + kh * a.sd.k.h, D, g);
-    row_load<DT, VEC>(vf, a.v, b * a.sd.v.b + jc * a.sd.v.t + kh * a.sd.v.h, D, g);
+    const int64_t ko = b * a.sd.k.b + jc * a.sd.k.t + kh * a.sd.k.h, vo = b * a.sd.v.b + jc * a.sd.v.t + kh * a.sd.v.h;
+    row_load<DT, VEC>(kf, a.k, ko, D, g);
+    row_load<DT, VEC>(vf, a.v, vo, D, g);
     const bool pad = j >= Tk || (a.m.pad && a.m.pad[b * Tk + jc]);
     f32x4_t ak[NS], av[NS];
 #pragma unroll
@@ -347,6 +449,13 @@ __global__ __launch_bounds__(64 * kNW) void attn_dkdv_f32(AttnF32 a, void *dk, v
         row_load<DT, VEC>(qf, a.q, q_off(h, i), D, g);
         row_load<DT, VEC>(gf, a.d_o, g_off(h, i), D, g);
     };
+    auto record = [&](int64_t h, int64_t i) {
+        RowRec x = a.rec[(b * Tq + clampq(i)) * a.Hq + h];
+        if (i >= Tq) x.lo = x.hi = 0;
+        return x;
+    };
+    auto sees = [&](const RowRec &x) { return !pad && j >= x.lo && j < x.hi; };
+    bool badq = false, badg = false;
     if (wave < n) load(wave);
     for (int e = wave; e < n; e += kNW) {
         const int64_t h = kh * group + e % group, i0 = (int64_t)(t0 + e / group) * kQT + 4 * g;
@@ -355,8 +464,7 @@ __global__ __launch_bounds__(64 * kNW) void attn_dkdv_f32(AttnF32 a, void *dk, v
 #pragma unroll
         for (int r = 0; r < 4; r++) {
             const int64_t i = clampq(i0 + r);
-            rec[r] = a.rec[(b * Tq + i) * a.Hq + h];
-            if (i0 + r >= Tq) rec[r].lo = rec[r].hi = 0;
+            rec[r] = record(h, i0 + r);
             qo[r] = q_off(h, i);
             go[r] = g_off(h, i);
         }
@@ -368,32 +476,67 @@ __global__ __launch_bounds__(64 * kNW) void attn_dkdv_f32(AttnF32 a, void *dk, v
                 gc[s] = col_load<DT>(a.d_o, go, 16 * s + c, D);
             }
         }
+        bool on[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) on[r] = sees(rec[r]);
+        const bool all = all_seen(on);
+        if constexpr (kEarly) {
+            if (!all) {
+                const Hidden hid(on, j < Tk);
+                badq |= hid.clear(qc);
+                badg |= hid.clear(gc);
+            }
+        }
         const f32x4_t sv = rows_dot(qf, kf), dp = rows_dot(gf, vf);
         if (e + kNW < n) load(e + kNW);
         float p[4], ds[4];
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-            const bool on = !pad && j >= rec[r].lo && j < rec[r].hi;
-            p[r] = on ? expf(sv[r] * a.scale - rec[r].lse) : 0.f;
-            ds[r] = on ? p[r] * (dp[r] - rec[r].delta) : 0.f;
+            p[r] = on[r] ? expf(sv[r] * a.scale - rec[r].lse) : 0.f;
+            ds[r] = on[r] ? p[r] * (dp[r] - rec[r].delta) : 0.f;
         }
 #pragma unroll
         for (int s = 0; s < NS; s++) {
-            f32x4_t x, y;
+            f32x4_t x[1], y[1];
             if constexpr (kEarly) {
-                x = qc[s];
-                y = gc[s];
+                x[0] = qc[s];
+                y[0] = gc[s];
             } else {
-                x = col_load<DT>(a.q, qo, 16 * s + c, D);
-                y = col_load<DT>(a.d_o, go, 16 * s + c, D);
+                x[0] = col_load<DT>(a.q, qo, 16 * s + c, D);
+                y[0] = col_load<DT>(a.d_o, go, 16 * s + c, D);
+                if (!all) {
+                    const Hidden hid(on, j < Tk);
+                    badq |= hid.clear(x);
+                    badg |= hid.clear(y);
+                }
             }
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                ak[s] = mfma4(x[r], ds[r], ak[s]);
-                av[s] = mfma4(y[r], p[r], av[s]);
+                ak[s] = mfma4(x[0][r], ds[r], ak[s]);
+                av[s] = mfma4(y[0][r], p[r], av[s]);
             }
         }
     }
+    auto again = [&](f32x4_t (&acc)[NS], const void *which, auto own, auto weight) {
+        for (int e = wave; e < n; e += kNW) {
+            const int64_t h = kh * group + e % group, i0 = (int64_t)(t0 + e / group) * kQT;
+            bool on[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) on[r] = sees(record(h, i0 + 4 * g + r));
+            if (!Hidden(on, j < Tk).cut) continue;
+#pragma unroll 1
+            for (int64_t i = i0; i < i0 + kQT; i++) {
+                const RowRec x = record(h, i);
+                const int64_t q0 = q_off(h, clampq(i)), g0 = g_off(h, clampq(i));
+                const float p = expf(dot4<DT>(a.q, q0, a.k, ko, D) * a.scale - x.lse);
+                add_not_finite<DT>(acc, which, own(q0, g0), sees(x), weight(p, x.delta, g0), D);
+            }
+        }
+    };
+    if (badq)
+        again(ak, a.q, [](int64_t q0, int64_t) { return q0; },
+              [&](float p, float delta, int64_t g0) { return p * (dot4<DT>(a.d_o, g0, a.v, vo, D) - delta); });
+    if (badg) again(av, a.d_o, [](int64_t, int64_t g0) { return g0; }, [](float p, float, int64_t) { return p; });
     constexpr int kL = 4 * kNW;
     const int r = threadIdx.x / kL;
     const int64_t to = ((b * Tk + kt * kQT + r) * a.Hkv + kh) * D;

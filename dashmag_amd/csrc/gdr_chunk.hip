@@ -227,6 +227,55 @@ __device__ __forceinline__ void gemm64_lds(Quad &acc, const float *A, FB fb, flo
     }
 }
 
+// Products with a triangular matrix (A[i][k], used where k <= i, or with UPPER where k >= i): the zeros of
+// its other half are multiplied like the rest, and 0 * inf is NaN, so a token's value that is not
+// finite would reach tokens that do not depend on it (the earlier ones forward). Such a product is NaN
+// somewhere; a workgroup that finds one takes the sum again term by term over the triangle alone
+// (finite inputs pay the test: 16 compares a lane and a barrier).
+__device__ __forceinline__ bool not_finite(const Quad &acc) {
+    bool bad = false;
+#pragma unroll
+    for (int ti = 0; ti < 2; ti++)
+#pragma unroll
+        for (int tj = 0; tj < 2; tj++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) bad |= !(fabsf(acc[ti][tj][r]) < INFINITY);
+    return bad;
+}
+// Whether any thread of the workgroup says so; a barrier must lie between two uses of sm (4 ints).
+__device__ __forceinline__ bool block_any(bool x, int *sm) {
+    const bool w = __any(x);
+    if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = w;
+    __syncthreads();
+    return (sm[0] | sm[1] | sm[2] | sm[3]) != 0;
+}
+// acc += A B over the triangle; fa, fb, TA and TB as gemm64's.
+template <bool TA, bool TB, bool UPPER, class FA, class FB>
+__device__ __forceinline__ void tri_sum(Quad &acc, FA fa, FB fb) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int i0 = (wave >> 1) * 32 + 4 * (lane >> 4), j0 = (wave & 1) * 32 + (lane & 15);
+#pragma unroll 1
+    for (int k = 0; k < kChunk; k++) {
+        float b[2];
+#pragma unroll
+        for (int tj = 0; tj < 2; tj++) {
+            const int j = j0 + 16 * tj;
+            b[tj] = TB ? at4(fb(k, j & ~3), j & 3) : at4(fb(j, k & ~3), k & 3);
+        }
+#pragma unroll
+        for (int ti = 0; ti < 2; ti++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int i = i0 + 16 * ti + r;
+                const float a = TA ? at4(fa(k, i & ~3), i & 3) : at4(fa(i, k & ~3), k & 3);
+                if (UPPER ? k >= i : k <= i) {
+                    acc[ti][0][r] = fmaf(a, b[0], acc[ti][0][r]);
+                    acc[ti][1][r] = fmaf(a, b[1], acc[ti][1][r]);
+                }
+            }
+    }
+}
+
 // f(row, column, values): rows row .. row + 3 of one column, for each tile of the quadrant.
 template <class F>
 __device__ __forceinline__ void each4(const Quad &acc, F f) {
@@ -287,8 +336,6 @@ struct Rows {
 // normalised, queries scaled; G; A and P = Q K^T o decay; T = (I + A)^-1; W and U.
 // T in f32 by 16 x 16 blocks: each diagonal block by column forward substitution (a wavefront a
 // block), the blocks below by doubling, T21 = -T22 (A21 T11).
-// Products run over whole chunks, as the reference's: a value that is not finite reaches every
-// row of its chunk.
 // ------------------------------------------------------------------------------------------
 
 // One wavefront's 16 x 16 block product over k = 16: A[i][k] at A, B[k][j] at B.
@@ -310,6 +357,7 @@ __global__ __launch_bounds__(256) void gdr_prep(GdrArgs a, GdrWs w, const void *
     __shared__ float4 smem[(2 * kPanels + 2 * kChunk * kMatS) / 4];
     __shared__ double G[kChunk];
     __shared__ float gam[kChunk], bet[kChunk], lam[kChunk];
+    __shared__ int flag[4];
     float *pan = (float *)smem, *Ts = pan + 2 * kPanels, *As = Ts + kChunk * kMatS;
     float *mm = pan;  // four 16 x 16 blocks, while no panel is in use
 
@@ -362,6 +410,7 @@ __global__ __launch_bounds__(256) void gdr_prep(GdrArgs a, GdrWs w, const void *
         put(vp, VP, x[2], 1.f, 1.f);
         if constexpr (BWD) put(dop, VP, x[3], 1.f, 1.f);
     }
+    if (tid < 4) flag[tid] = 0;
     if (wave == 0) {
         const bool ok = lane < len;
         double x = ok ? ld_any(a.g_dt, a.g, g_at(a, tok0 + lane, h)) : 0.f;
@@ -422,6 +471,12 @@ __global__ __launch_bounds__(256) void gdr_prep(GdrArgs a, GdrWs w, const void *
                 if constexpr (BWD) Ag[i * kChunk + j] = av;
             }
     __syncthreads();
+    bool bad = false;  // T is not finite somewhere
+    auto note = [&](const f32x4_t &v) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) bad |= !(fabsf(v[r]) < INFINITY);
+        return v;
+    };
     {
         // diagonal block b = wave, lane c holding column c of its inverse:
         // T[i][c] = [i == c] - sum_{x < i} A[i][x] T[x][c]
@@ -438,6 +493,7 @@ __global__ __launch_bounds__(256) void gdr_prep(GdrArgs a, GdrWs w, const void *
                     if (x4 + e < i) sp[e] += at4(a4, e) * tc[x4 + e];
             }
             tc[i] = (i == c ? 1.f : 0.f) - ((sp[0] + sp[1]) + (sp[2] + sp[3]));
+            bad |= !(fabsf(tc[i]) < INFINITY);
         }
         if (lane < 16) {
 #pragma unroll
@@ -460,7 +516,7 @@ __global__ __launch_bounds__(256) void gdr_prep(GdrArgs a, GdrWs w, const void *
         if (wave < 2) put(mm + wave * 320, 20, block16(blk(As, bi1, bj1), kMatS, blk(Ts, bj1, bj1), kMatS, z), 1.f);
         __syncthreads();
         if (wave < 2)
-            put(blk(Ts, bi1, bj1), kMatS, block16(blk(Ts, bi1, bi1), kMatS, mm + wave * 320, 20, z), -1.f);
+            put(blk(Ts, bi1, bj1), kMatS, note(block16(blk(Ts, bi1, bi1), kMatS, mm + wave * 320, 20, z)), -1.f);
         __syncthreads();
         // the lower-left quarter, wavefront w its block (2 + w / 2, w % 2)
         const int bi = 2 + (wave >> 1), bj = wave & 1;
@@ -471,9 +527,21 @@ __global__ __launch_bounds__(256) void gdr_prep(GdrArgs a, GdrWs w, const void *
         x = z;
         for (int kb = 2; kb <= bi; kb++)
             x = block16(blk(Ts, bi, kb), kMatS, mm + (2 * (kb - 2) + bj) * 320, 20, x);
-        put(blk(Ts, bi, bj), kMatS, x, -1.f);
+        put(blk(Ts, bi, bj), kMatS, note(x), -1.f);
+        if (__any(bad) && lane == 0) flag[wave] = 1;
     }
     __syncthreads();
+    if (flag[0] | flag[1] | flag[2] | flag[3]) {
+        // a column a thread, row after row, so that a row comes from the ones before it alone
+        if (tid < kChunk) {
+            for (int i = 0; i < kChunk; i++) {
+                float s = i == tid ? 1.f : 0.f;
+                for (int x = tid; x < i; x++) s -= As[i * kMatS + x] * Ts[x * kMatS + tid];
+                Ts[i * kMatS + tid] = s;
+            }
+        }
+        __syncthreads();
+    }
     if constexpr (BWD) {
         float *Tg = w.Tm + ch * kChunk * kChunk;
         for (int x = tid; x < kChunk * kChunk / 4; x += 256)
@@ -481,29 +549,35 @@ __global__ __launch_bounds__(256) void gdr_prep(GdrArgs a, GdrWs w, const void *
     }
     // W = T (beta gamma K), U = T (beta V); W as the state pass's rows and, for the backward's,
     // transposed; U transposed
-    for (int x0 = 0; x0 < KP; x0 += 64) {
-        Quad acc;
-        zero_quad(acc);
-        gemm64_lds<true>(acc, Ts, [&](int j, int c) {
-            return scaled(*(const float4 *)(kn + j * KP + x0 + c), bet[j] * gam[j]);
-        }, pan);
-        each4(acc, [&](int i, int x, const f32x4_t &v) {
-            float *W = w.W + ch * kChunk * KP;
+    auto wu = [&](auto product) {
+        bool bad = false;
+        for (int x0 = 0; x0 < KP; x0 += 64) {
+            Quad acc;
+            zero_quad(acc);
+            product(acc, [&](int j, int c) {
+                return scaled(*(const float4 *)(kn + j * KP + x0 + c), bet[j] * gam[j]);
+            });
+            bad |= not_finite(acc);
+            each4(acc, [&](int i, int x, const f32x4_t &v) {
+                float *W = w.W + ch * kChunk * KP;
 #pragma unroll
-            for (int r = 0; r < 4; r++) W[(i + r) * KP + x0 + x] = v[r];
-            if constexpr (BWD) *(float4 *)(w.WT + ch * kChunk * KP + (x0 + x) * kChunk + i) = as_f4(v);
-        });
-    }
-    for (int y0 = 0; y0 < VP; y0 += 64) {
-        Quad acc;
-        zero_quad(acc);
-        gemm64_lds<true>(acc, Ts, [&](int j, int c) {
-            return scaled(*(const float4 *)(vp + j * VP + y0 + c), bet[j]);
-        }, pan);
-        each4(acc, [&](int i, int y, const f32x4_t &v) {
-            *(float4 *)(w.UT + ch * kChunk * VP + (y0 + y) * kChunk + i) = as_f4(v);
-        });
-    }
+                for (int r = 0; r < 4; r++) W[(i + r) * KP + x0 + x] = v[r];
+                if constexpr (BWD) *(float4 *)(w.WT + ch * kChunk * KP + (x0 + x) * kChunk + i) = as_f4(v);
+            });
+        }
+        for (int y0 = 0; y0 < VP; y0 += 64) {
+            Quad acc;
+            zero_quad(acc);
+            product(acc, [&](int j, int c) { return scaled(*(const float4 *)(vp + j * VP + y0 + c), bet[j]); });
+            bad |= not_finite(acc);
+            each4(acc, [&](int i, int y, const f32x4_t &v) {
+                *(float4 *)(w.UT + ch * kChunk * VP + (y0 + y) * kChunk + i) = as_f4(v);
+            });
+        }
+        return bad;
+    };
+    if (block_any(wu([&](Quad &acc, auto f) { gemm64_lds<true>(acc, Ts, f, pan); }), flag))
+        wu([&](Quad &acc, auto f) { tri_sum<false, true, false>(acc, Rows{Ts, kMatS}, f); });
     // (lam K)^T
     float *KT = w.KT + ch * kChunk * KP;
     const int ld = (int)KP;
@@ -685,22 +759,30 @@ __global__ __launch_bounds__(256) void gdr_output(GdrArgs a, GdrWs w, void *out)
     const int y0 = blockIdx.y * 64;
     __shared__ float4 smem[2 * kPanels / 4];
     __shared__ float gam[kChunk];
+    __shared__ int flag[4];
     if (threadIdx.x < kChunk) gam[threadIdx.x] = expf((float)w.G[ch * kChunk + threadIdx.x]);
     Quad acc;
-    zero_quad(acc);
-    gemm64<false, false>(acc, Rows{w.qn + ch * kChunk * KP, KP}, Rows{w.ScT + (ch * VP + y0) * KP, KP},
-                         (int)KP, (float *)smem);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const Rows fp{w.P + ch * kChunk * kChunk, kChunk}, fv{w.VnT + (ch * VP + y0) * kChunk, kChunk};
+    auto from_state = [&] {
+        zero_quad(acc);
+        gemm64<false, false>(acc, Rows{w.qn + ch * kChunk * KP, KP}, Rows{w.ScT + (ch * VP + y0) * KP, KP},
+                             (int)KP, (float *)smem);
 #pragma unroll
-    for (int ti = 0; ti < 2; ti++)
+        for (int ti = 0; ti < 2; ti++)
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const float gm = gam[(wave >> 1) * 32 + ti * 16 + 4 * (lane >> 4) + r];
-            acc[ti][0][r] *= gm;
-            acc[ti][1][r] *= gm;
-        }
-    gemm64<false, false>(acc, Rows{w.P + ch * kChunk * kChunk, kChunk},
-                         Rows{w.VnT + (ch * VP + y0) * kChunk, kChunk}, kChunk, (float *)smem);
+            for (int r = 0; r < 4; r++) {
+                const float gm = gam[(wave >> 1) * 32 + ti * 16 + 4 * (lane >> 4) + r];
+                acc[ti][0][r] *= gm;
+                acc[ti][1][r] *= gm;
+            }
+    };
+    from_state();
+    gemm64<false, false>(acc, fp, fv, kChunk, (float *)smem);
+    if (block_any(not_finite(acc), flag)) {
+        from_state();
+        tri_sum<false, false, false>(acc, fp, fv);
+    }
     each4(acc, [&](int i, int y, const f32x4_t &v) {
 #pragma unroll
         for (int r = 0; r < 4; r++)
@@ -721,6 +803,7 @@ __global__ __launch_bounds__(256) void gdr_bwd_local(GdrArgs a, GdrWs w) {
     const int vt = (int)(VP / 64), job = blockIdx.y;
     __shared__ float4 smem[2 * kPanels / 4];
     __shared__ float gam[kChunk];
+    __shared__ int flag[4];
     if (threadIdx.x < kChunk) gam[threadIdx.x] = expf((float)w.G[ch * kChunk + threadIdx.x]);
     __syncthreads();
     const int y0 = (job % vt) * 64;
@@ -728,7 +811,12 @@ __global__ __launch_bounds__(256) void gdr_bwd_local(GdrArgs a, GdrWs w) {
     Quad acc;
     zero_quad(acc);
     if (job < vt) {
-        gemm64<true, true>(acc, Rows{w.P + ch * kChunk * kChunk, kChunk}, dO, kChunk, (float *)smem);
+        const Rows fp{w.P + ch * kChunk * kChunk, kChunk};
+        gemm64<true, true>(acc, fp, dO, kChunk, (float *)smem);
+        if (block_any(not_finite(acc), flag)) {
+            zero_quad(acc);
+            tri_sum<true, true, true>(acc, fp, dO);
+        }
         each4(acc, [&](int j, int y, const f32x4_t &v) {
             *(float4 *)(w.dvlT + (ch * VP + y0 + y) * kChunk + j) = as_f4(v);
         });
@@ -925,6 +1013,7 @@ __global__ __launch_bounds__(256) void gdr_bwd_rows(GdrArgs a, GdrWs w, void *dv
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, kt = (int)(KP / 64);
     __shared__ float4 smem[2 * kPanels / 4];
     __shared__ float bet[kChunk], bg[kChunk], red[4][2 * kChunk];
+    __shared__ int flag[4];
     float *pan = (float *)smem;
     if (tid < kChunk) {
         bet[tid] = tid < len ? ld_any(a.beta_dt, a.beta, b_at(a, tok0 + tid, h)) : 0.f;
@@ -938,7 +1027,12 @@ __global__ __launch_bounds__(256) void gdr_bwd_rows(GdrArgs a, GdrWs w, void *dv
         const float *vp = w.vp + ch * kChunk * VP + y0;
         Quad acc;
         zero_quad(acc);
-        gemm64<true, false>(acc, ft, Rows{w.dVnT + (ch * VP + y0) * kChunk, kChunk}, kChunk, pan);
+        const Rows fd{w.dVnT + (ch * VP + y0) * kChunk, kChunk};
+        gemm64<true, false>(acc, ft, fd, kChunk, pan);
+        if (block_any(not_finite(acc), flag)) {
+            zero_quad(acc);
+            tri_sum<true, false, true>(acc, ft, fd);
+        }
 #pragma unroll
         for (int ti = 0; ti < 2; ti++)
 #pragma unroll
@@ -967,8 +1061,14 @@ __global__ __launch_bounds__(256) void gdr_bwd_rows(GdrArgs a, GdrWs w, void *dv
     zero_quad(xw);
     zero_quad(xe);
     gemm64<false, true>(xq, fp, fk, kChunk, pan);
-    gemm64<false, true>(xe, fa, fk, kChunk, pan);
     gemm64<true, true>(xk, fp, fq, kChunk, pan);
+    if (block_any(not_finite(xq) || not_finite(xk), flag)) {
+        zero_quad(xq);
+        zero_quad(xk);
+        tri_sum<false, true, false>(xq, fp, fk);
+        tri_sum<true, true, true>(xk, fp, fq);
+    }
+    gemm64<false, true>(xe, fa, fk, kChunk, pan);
     gemm64<true, true>(xk, fa, [&](int j, int c) {
         return scaled(*(const float4 *)(kn + j * KP + c), bet[j]);
     }, kChunk, pan);

@@ -77,3 +77,46 @@ def test_matches_oracle(dtype, dk, dv, lens, h, l2norm, states):
         rel = errors(host(x), e)[1]
         print(f"  {name}: rel {rel:.2e}")
         assert rel <= tol, name
+
+
+@pytest.mark.parametrize("dtype,dk,dv", [(torch.float32, 128, 128), (torch.float32, 20, 36),
+                                         (torch.bfloat16, 136, 72)])
+@pytest.mark.parametrize("what", ["q", "k", "v", "beta", "g", "do"])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_tokens_depend_on_earlier_ones_alone(what, dtype, dk, dv, value):
+    """A token's value that is not finite does not reach the results that do not depend on it, within
+    its chunk either: forward, the outputs of the tokens before it (of every other token for a query);
+    backward, with a gradient or query at fault, dv of the tokens after it and dq of every other; with
+    a value, dq of the tokens before it, dv and the initial state's gradient. Bounds as above (such a
+    chunk's sums run in another order)."""
+    T, H, x = 150, 2, 90
+    print(f"case {what} {value} {dtype} {dk}x{dv}", flush=True)
+    q = syn.l2norm(syn.normal(71, (1, T, H, dk), "cuda")).to(dtype)
+    k = syn.l2norm(syn.normal(72, (1, T, H, dk), "cuda")).to(dtype)
+    v, do = (syn.normal(s, (1, T, H, dv), "cuda").to(dtype) for s in (73, 74))
+    g = -torch.nn.functional.softplus(syn.normal(75, (1, T, H), "cuda"))
+    beta = torch.sigmoid(syn.normal(76, (1, T, H), "cuda"))
+    h0 = syn.normal(77, (1, H, dk, dv), "cuda", std=0.1)
+    opts = dm.ChunkGatedDeltaOptions(output_final_state=True)
+    bad = dict(q=q.clone(), k=k.clone(), v=v.clone(), g=g.clone(), beta=beta.clone(), do=do.clone())
+    bad[what][0, x, 0] = value
+
+    def step(q, k, v, g, beta, do):
+        out, fin = dm.chunk_gated_delta_rule(q, k, v, g, beta, h0, None, opts)
+        gr = dm.chunk_gated_delta_rule_backward(q, k, v, g, beta, h0, None, do, None, opts)
+        return dict(out=out, fin=fin, dq=gr[0], dv=gr[2], dh0=gr[5])
+    want, got = step(q, k, v, g, beta, do), step(**bad)
+    before, after = slice(0, x), slice(x + 1, T)
+    same = {"q": dict(out=(before, after), fin=(slice(None),), dq=(before, after), dv=(after,)),
+            "k": dict(out=(before,)), "beta": dict(out=(before,)), "g": dict(out=(before,)),
+            "v": dict(out=(before,), dq=(before,), dv=(slice(None),), dh0=(slice(None),)),
+            "do": dict(out=(slice(None),), fin=(slice(None),), dq=(before, after), dv=(after,))}[what]
+    tol = 4e-6 if dtype == torch.float32 else 4e-3
+    for name, parts in same.items():
+        for part in parts:
+            a, e = host(got[name][:, part]), host(want[name][:, part])
+            assert np.isfinite(a).all(), (name, part)
+            assert errors(a, e)[1] <= tol, (name, part)
+    for name in want:  # the other head
+        h = 1 if name in ("fin", "dh0") else 2
+        assert torch.equal(got[name].select(h, 1), want[name].select(h, 1)), name

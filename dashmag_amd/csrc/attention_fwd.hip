@@ -484,10 +484,14 @@ extern "C" int dm_debug_trace_fwd(void *host, size_t bytes) {
 // keys of 8 heads of 128: 152 -> 28; unmasked 6144 of width 64 (192 equal items) are as fast whole.
 static size_t fwd_split(const dm_attention_desc *d, char *base, FwdSplit *sp) {
     constexpr int kCUs = 256, kMinTiles = 6, kSegCost = 3, kMergeCost = 4;
+    sp->nseg = 0;
+    // the size query comes here before the call's checks: sizes of any value, each bounded before a product
+    if (d->b <= 0 || d->hq <= 0 || d->tq <= 0 || d->b >= kCUs || d->hq >= kCUs || d->tq >= (1 << 30) ||
+        d->tk >= (1 << 30))
+        return 0;
     const int64_t per = 32 * (d->d == 256 ? fwd_waves<256>() : fwd_waves<128>());
     const int64_t nt = (d->tq + per - 1) / per, rows = d->hq * d->b;
-    sp->nseg = 0;
-    if (nt * rows == 0 || nt * rows >= kCUs || d->tk <= kMinTiles * kFwdN) return 0;
+    if (nt * rows >= kCUs || d->tk <= kMinTiles * kFwdN) return 0;
     if (d->mask_kind == DM_MASK_PACKED && d->nseq > 2) return 0;
     // Key tiles of each query tile, from the mask's closed form. Offsets lie on the device: two packed
     // sequences are taken for equal ones, and calls of more run whole (equal lengths taken for one

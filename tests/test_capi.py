@@ -151,3 +151,21 @@ def test_noalloc_decode_refuses_calls_beyond_its_scratch():
     rc = lb.dm_attention_decode_noalloc(ctypes.byref(d), None, None, None, None, None, None)
     assert rc == _lib.DM_ERR_REFUSED
     assert _lib.last_error().startswith("attention_decode: the call needs")
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("b,tq,hq,tk", [
+    (1, -1000, 8, 4096), (-1, 100000, 1, 4096), (-1, 1000, 1, 4096), (-3, -70000, 1, 4096), (1, 1000, -4, 4096),
+    (1, 1000, 8, -4096), (1 << 40, 1 << 20, 1 << 24, 4096), (1 << 62, 64, 4, 4096), (3, (1 << 63) - 1, 1, 4096),
+    (1, 1000, 8, 1 << 62)])
+def test_forward_workspace_of_refused_sizes(b, tq, hq, tk, d):
+    """The forward's size query answers 0 for sizes that no call has: a caller asks before the call that
+    refuses it, so the query neither fails nor names a size."""
+    x = _lib.AttentionDesc(b=b, tq=tq, tk=tk, hq=hq, hkv=1, d=d, dtype=_lib.DM_BF16, mask_kind=_lib.DM_MASK_NONE)
+    for causal in (0, 1):
+        x.options.causal = causal
+        assert _lib.lib().dm_attention_fwd_workspace(ctypes.byref(x)) == 0
+    if min(b, tq, hq, tk) < 0:
+        assert _lib.lib().dm_attention_fwd(ctypes.byref(x), None, None, None, None, None, None, 0,
+                                           None) == _lib.DM_ERR_REFUSED
+        assert _lib.last_error() == "attention: negative dimension"

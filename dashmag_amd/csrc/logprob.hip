@@ -504,9 +504,9 @@ static int lt_gemm(hipStream_t st, bool ta, bool tb, int64_t m, int64_t n, int64
     return DM_OK;
 }
 
-// Rows of the loss's backward whose chunk of logits' gradients is held for one weight-gradient
-// product (at 8192 columns in bf16 256 MB at most).
-constexpr int64_t kLceGroup = 16384;
+// Bytes of logits' gradients that the loss's backward holds for one weight-gradient product at most
+// (16384 rows of 8192 columns in bf16).
+constexpr int64_t kLceGroup = 256 << 20;
 
 struct LpPlan {
     int64_t block, chunk;  // rows per block, vocabulary tokens per chunk
@@ -518,8 +518,9 @@ struct LpPlan {
 
 // What a call holds: grad (the log-probability's softmax weights, two bf16 parts or f32),
 // dz (the loss's logits gradient of a group of row blocks, bf16 or f32), and the loss's f32 gradient
-// accumulators when the gradients' dtype is not f32: the hidden's, and a chunk of the weight's.
-static LpPlan lp_plan(const dm_logprob_desc *d, bool grad, bool dz, bool gh32, bool gw32) {
+// accumulators when the gradients' dtype is not f32: the hidden's, and with gw (its gradient is wanted)
+// a chunk of the weight's.
+static LpPlan lp_plan(const dm_logprob_desc *d, bool grad, bool dz, bool gw) {
     LpPlan p{};
     const int64_t nb = d->n > 0 ? (d->n + d->row_chunk - 1) / d->row_chunk : 1;
     p.block = std::max<int64_t>(1, (d->n + nb - 1) / nb);
@@ -528,8 +529,16 @@ static LpPlan lp_plan(const dm_logprob_desc *d, bool grad, bool dz, bool gh32, b
     p.chunk = d->vocab_chunk > 0 ? d->vocab_chunk : kLpMaxChunk;
     p.chunk = std::min<int64_t>({p.chunk, kLpMaxChunk, std::max<int64_t>(d->v, 1)});
     p.bf16 = d->hidden_dtype == DM_BF16 && d->weight_dtype == DM_BF16;
-    p.group = std::max<int64_t>(1, kLceGroup / p.block) * p.block;
-    p.group = std::min(p.group, std::max<int64_t>(d->n, 1));
+    // In bf16 the group takes no more than a block in f32 does, or with the weight's gradient than the
+    // f32 accumulator of all of it that the group stands for. In f32 arithmetic a block's product is
+    // long against reading and writing its accumulator, and there is little to group for.
+    p.group = p.block;
+    if (p.bf16 && dz) {
+        const double row = 2. * (double)p.chunk;
+        double room = 2. * row * (double)p.block;
+        if (gw) room = std::max(room, std::min((double)kLceGroup, 4. * (double)(d->v - p.chunk) * (double)d->d));
+        p.group = std::min((int64_t)(room / (row * (double)p.block)) * p.block, std::max<int64_t>(d->n, 1));
+    }
     const int64_t n1 = std::max<int64_t>(d->n, 1);
     size_t o = 0;
     p.off_bits = o;
@@ -548,9 +557,9 @@ static LpPlan lp_plan(const dm_logprob_desc *d, bool grad, bool dz, bool gh32, b
     p.off_coef = o;
     if (dz) o += align_up((size_t)LC_COUNT * n1 * 4);
     p.off_gh = o;
-    if (gh32) o += align_up((size_t)d->n * d->d * 4);
+    if (dz && d->hidden_dtype != DM_F32) o += align_up((size_t)d->n * d->d * 4);
     p.off_gw = o;
-    if (gw32) o += align_up((size_t)p.chunk * d->d * 4);
+    if (gw && d->weight_dtype != DM_F32) o += align_up((size_t)p.chunk * d->d * 4);
     p.off_lt = o;
     o += kLtWorkspace;
     p.total = o;
@@ -726,7 +735,7 @@ extern "C" {
 
 size_t dm_chosen_logprob_workspace(const dm_logprob_desc *d, int with_grad) {
     if (lp_check("chosen_logprob", d, false) != DM_OK) return 0;
-    return lp_plan(d, with_grad != 0, false, false, false).total;
+    return lp_plan(d, with_grad != 0, false, false).total;
 }
 
 int dm_chosen_logprob(const dm_logprob_desc *d, const void *hidden, const void *weight,
@@ -738,7 +747,7 @@ int dm_chosen_logprob(const dm_logprob_desc *d, const void *hidden, const void *
     std::vector<uint32_t> bits;
     if (lp_bits(op, d, masked, n_masked, bits) < 0) return DM_ERR_REFUSED;
     const bool want_grad = grad != nullptr;
-    const LpPlan p = lp_plan(d, want_grad, false, false, false);
+    const LpPlan p = lp_plan(d, want_grad, false, false);
     if (workspace_bytes < p.total)
         return refuse(op + ": the workspace is smaller than dm_chosen_logprob_workspace");
     if (d->n == 0) return DM_OK;
@@ -769,9 +778,8 @@ int dm_chosen_logprob(const dm_logprob_desc *d, const void *hidden, const void *
 
 size_t dm_linear_cross_entropy_workspace(const dm_lce_desc *d, int backward) {
     if (lce_check(d) != DM_OK) return 0;
-    const bool f32 = d->lp.hidden_dtype == DM_F32;
     // backward 1: both gradients; 2: the hidden's alone (no weight-gradient accumulator)
-    return lp_plan(&d->lp, false, backward != 0, backward && !f32, backward == 1 && !f32).total;
+    return lp_plan(&d->lp, false, backward != 0, backward == 1).total;
 }
 
 int dm_linear_cross_entropy_fwd(const dm_lce_desc *d, const void *hidden, const void *weight,
@@ -784,7 +792,7 @@ int dm_linear_cross_entropy_fwd(const dm_lce_desc *d, const void *hidden, const 
     std::vector<uint32_t> bits;
     const int64_t nmask = lp_bits(op, lp, masked, n_masked, bits);
     if (nmask < 0) return DM_ERR_REFUSED;
-    const LpPlan p = lp_plan(lp, false, false, false, false);
+    const LpPlan p = lp_plan(lp, false, false, false);
     if (workspace_bytes < p.total)
         return refuse(op + ": the workspace is smaller than dm_linear_cross_entropy_workspace");
     if (lp->n == 0) return DM_OK;
@@ -817,9 +825,9 @@ int dm_linear_cross_entropy_bwd(const dm_lce_desc *d, const void *hidden, const 
     const int64_t nmask = lp_bits(op, lp, masked, n_masked, bits);
     if (nmask < 0) return DM_ERR_REFUSED;
     const bool f32 = lp->hidden_dtype == DM_F32;
-    // the weight-gradient accumulator (16-bit inputs) is reserved only when that gradient is
-    // asked for: dm_linear_cross_entropy_workspace(desc, 2) sizes a call without it
-    const LpPlan p = lp_plan(lp, false, true, !f32, !f32 && grad_weight != nullptr);
+    // what the weight's gradient takes is reserved only when it is asked for:
+    // dm_linear_cross_entropy_workspace(desc, 2) sizes a call without it
+    const LpPlan p = lp_plan(lp, false, true, grad_weight != nullptr);
     if (workspace_bytes < p.total)
         return refuse(op + ": the workspace is smaller than dm_linear_cross_entropy_workspace");
     hipStream_t st = (hipStream_t)stream;
@@ -842,7 +850,7 @@ int dm_linear_cross_entropy_bwd(const dm_lce_desc *d, const void *hidden, const 
     // their gradient, a block of rows after another into G [rows of the group, chunk]; then
     // grad_hidden += G W_c, and grad_weight_c = G^T H over all of the group's rows in one product.
     // The chunk is the outer loop so that the weight's gradient is summed within a product and
-    // written once, in its own dtype (bf16 with at most one group of rows): accumulated per row
+    // written once, in its own dtype (bf16 with one group of rows): accumulated per row
     // block in f32 over the whole vocabulary, 4096 rows of 4096 by 151936 tokens moved 10 GB more
     // (of which 3.7 GB, 720 us, rounded the sum), and its products of 2048 rows each took 165 us a
     // chunk where one of 4096 takes 250. With more groups an f32 chunk accumulates.

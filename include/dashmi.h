@@ -402,8 +402,11 @@ int dm_chosen_logprob(const dm_logprob_desc *desc, const void *hidden, const voi
  * LinearCrossEntropyBackend::linear_cross_entropy (loss.rs:134-160; the written-out backward is
  * always taken, as with a weight that trains). The workspace query's `backward`: 0 for the
  * forward, 1 for a backward with both gradients, 2 for a backward without grad_weight (a frozen
- * output weight: no f32 accumulator for a chunk of it is reserved; the backward then refuses a
- * non-NULL grad_weight with that smaller workspace). */
+ * output weight: a block of rows' logits and as many bytes for their gradient are held, and no
+ * f32 accumulator for a chunk of the weight; the backward then refuses a non-NULL grad_weight with
+ * that smaller workspace). From bf16 inputs 1 holds the logits' gradients of several blocks of rows,
+ * so that row_chunk bounds the f32 logits alone: up to 256 MB, and no more than V x D f32 values
+ * take. */
 size_t dm_linear_cross_entropy_workspace(const dm_lce_desc *desc, int backward);
 int dm_linear_cross_entropy_fwd(const dm_lce_desc *desc, const void *hidden, const void *weight,
                                 const int64_t *targets, const uint32_t *masked, int64_t n_masked,

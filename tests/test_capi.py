@@ -169,3 +169,20 @@ def test_forward_workspace_of_refused_sizes(b, tq, hq, tk, d):
         assert _lib.lib().dm_attention_fwd(ctypes.byref(x), None, None, None, None, None, None, 0,
                                            None) == _lib.DM_ERR_REFUSED
         assert _lib.last_error() == "attention: negative dimension"
+
+
+@pytest.mark.parametrize("dtype", [_lib.DM_BF16, _lib.DM_F16, _lib.DM_F32])
+@pytest.mark.parametrize("n,row_chunk,v,d", [(16384, 1, 50000, 64), (40000, 3072, 151936, 4096), (40000, 100, 8192, 4096),
+                                             (3000, 3072, 151936, 64), (1000, 7, 300, 8), (0, 3072, 1000, 64)])
+def test_loss_workspace_bounds(dtype, n, row_chunk, v, d):
+    """What the loss's backward takes besides its inputs' f32 copies: without the weight's gradient the
+    logits of a block of rows, as much for their gradient and a few values a row; with it, no more than an f32 weight
+    gradient besides (f32: nothing)."""
+    lp = _lib.LogprobDesc(n=n, v=v, d=d, hidden_dtype=dtype, weight_dtype=dtype, vocab_chunk=0, row_chunk=row_chunk)
+    x = _lib.LceDesc(lp=lp)
+    frozen, both = (_lib.lib().dm_linear_cross_entropy_workspace(ctypes.byref(x), m) for m in (2, 1))
+    block = -(-n // -(-n // row_chunk)) if n else 1
+    chunk = min(v, 8192)
+    copies = {_lib.DM_BF16: n * d, _lib.DM_F16: 2 * n * d + v * d, _lib.DM_F32: 0}[dtype] * 4
+    assert frozen <= (64 << 20) + copies + 2 * block * chunk * 4 + 64 * max(n, 1) + v // 8 + 16 * 256
+    assert both <= frozen + (0 if dtype == _lib.DM_F32 else v * d * 4 + 256)

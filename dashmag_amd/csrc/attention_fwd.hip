@@ -478,12 +478,19 @@ extern "C" int dm_debug_trace_fwd(void *host, size_t bytes) {
 // long as its longest: 96 key tiles of 64 for the last of 6144 causal queries, where the chip's share
 // is 36. Of the segment lengths that cut the longest item in up to 16, the one is taken whose
 // workgroups, laid on 256 compute units longest first, end earliest, each workgroup costing
-// kSegCost tiles besides its own (its start, its partial outputs) and the split kMergeCost (the
-// merge). Measured, before and after: 6144 causal queries of 8 heads, width 64: 117 -> 75 us; width 128, 2048
-// queries: 58 -> 35, 4096: 108 -> 65, 6144: 155 -> 110; width 256, 2048: 92 -> 56; 16 queries against 8192
-// keys of 8 heads of 128: 152 -> 28; unmasked 6144 of width 64 (192 equal items) are as fast whole.
+// kSegCost tiles besides its own (its start, its partial outputs), the merge's launch kMergeCost (a
+// tile at width 256 takes longer) and the partial outputs' way through memory a tile per 64 workgroups of
+// 128 KB. Past two workgroups a unit they are taken to run in rounds, and cuts of more than
+// four (128 MB of partial outputs) are left out. (Charged the launch alone, and their even share past two
+// a unit, cuts far too fine were taken: 4594 unmasked queries of 8 heads of 128, 576 workgroups, took 142
+// us and take 117 in 432 or whole.) Of 45 calls of the three widths, each forced into up to ten cuts,
+// none takes longer by this rule than whole, and all together 1.8% longer than in the best of the cuts.
+// Measured, whole and split: 6144 causal queries of 8 heads, width 64: 114 -> 72 us; width 128, 2048
+// queries: 57 -> 33, 4096: 104 -> 60, 6144: 152 -> 107; width 256, 2048: 91 -> 52; 16 queries against
+// 8192 keys of 32 heads of 128: 152 -> 32; 51456 unmasked queries of one head of 64: 915 -> 731; unmasked
+// 6144 of 8 heads of 64 (192 equal items) are as fast whole.
 static size_t fwd_split(const dm_attention_desc *d, char *base, FwdSplit *sp) {
-    constexpr int kCUs = 256, kMinTiles = 6, kSegCost = 3, kMergeCost = 4;
+    constexpr int kCUs = 256, kMinTiles = 6, kSegCost = 3;
     sp->nseg = 0;
     // the size query comes here before the call's checks: sizes of any value, each bounded before a product
     if (d->b <= 0 || d->hq <= 0 || d->tq <= 0 || d->b >= kCUs || d->hq >= kCUs || d->tq >= (1 << 30) ||
@@ -493,40 +500,52 @@ static size_t fwd_split(const dm_attention_desc *d, char *base, FwdSplit *sp) {
     const int64_t nt = (d->tq + per - 1) / per, rows = d->hq * d->b;
     if (nt * rows >= kCUs || d->tk <= kMinTiles * kFwdN) return 0;
     if (d->mask_kind == DM_MASK_PACKED && d->nseq > 2) return 0;
-    // Key tiles of each query tile, from the mask's closed form. Offsets lie on the device: two packed
-    // sequences are taken for equal ones, and calls of more run whole (equal lengths taken for one
-    // sequence, 4 x 1536 causal tokens of 8 heads of 64, took 54 us against 36 whole; 5000, 500, 400 and
-    // 244 taken for equal ones 143 against 131).
-    MaskInfo m = mask_info(d);
-    const int64_t ns = m.kind == DM_MASK_PACKED ? std::max<int64_t>(d->nseq, 1) : 1;
-    m.kind = DM_MASK_NONE;
-    m.tq = (d->tq + ns - 1) / ns;
-    m.tk = (d->tk + ns - 1) / ns;
-    const int ntiles = (int)nt;
+    const int ntiles = (int)nt, kMergeCost = d->d == 256 ? 3 : 4;
+    // Key tiles of each query tile, from the mask's closed form for one sequence. Offsets lie on the
+    // device: two packed sequences are planned halfway between one and two of one length, and split where
+    // that promises a quarter. (6144 causal tokens of 8 heads of 128, whole, as two equal ones and so: 4096
+    // and 2048 107, 121 and 93 us; 5900 and 244 171, 138 and 123; 3072 twice 85, 78 and 86.) Calls of more
+    // run whole (4 x 1536 causal tokens of 8 heads of 64 taken for one sequence took 54 us against 36).
+    const bool two = d->mask_kind == DM_MASK_PACKED && d->nseq == 2;
+    MaskInfo m = mask_info(d), half = m;
+    m.kind = half.kind = DM_MASK_NONE;
+    half.tq = (d->tq + 1) / 2;
+    half.tk = (d->tk + 1) / 2;
     int n[kSplitTiles], most = 0;
     for (int t = 0; t < ntiles; t++) {
-        int64_t lo, hi, x;
         const int64_t q0 = (ntiles - 1 - t) * per, q1 = std::min(q0 + per, d->tq) - 1;
-        row_bounds(m, q0 % m.tq, &lo, &x);
-        row_bounds(m, q1 % m.tq, &x, &hi);
-        lo += q0 / m.tq * m.tk;
-        hi += q1 / m.tq * m.tk;
+        int64_t lo, hi, x;
+        row_bounds(m, q0, &lo, &x);
+        row_bounds(m, q1, &x, &hi);
         n[t] = (int)std::max<int64_t>((hi - lo + kFwdN - 1) / kFwdN, 1);
+        if (two) {
+            row_bounds(half, q0 % half.tq, &lo, &x);
+            row_bounds(half, q1 % half.tq, &x, &hi);
+            lo += q0 / half.tq * half.tk;
+            hi += q1 / half.tq * half.tk;
+            n[t] = (n[t] + (int)std::max<int64_t>((hi - lo + kFwdN - 1) / kFwdN, 1)) / 2;
+        }
         most = std::max(most, n[t]);
     }
-    // the time, in tiles, of segments of at most `steps`
+    // the time of segments of at most `steps`, in sixteenths of a tile (-1: too many of them)
     auto ends = [&](int steps) -> int64_t {
         std::pair<int, int64_t> len[kSplitTiles];  // length, how many
-        int64_t count = 0, total = 0;
+        int64_t count = 0;
         for (int t = 0; t < ntiles; t++) {
             const int ns = (n[t] + steps - 1) / steps;
             len[t] = {(n[t] + ns - 1) / ns + kSegCost, ns * rows};
             count += len[t].second;
-            total += len[t].second * len[t].first;
         }
-        if (count > 2 * kCUs) return total / kCUs + steps / 4;
+        if (count > 4 * kCUs) return -1;
         std::sort(len, len + ntiles, [](auto &a, auto &b) { return a.first > b.first; });
+        const int64_t merge = steps < most ? 16 * kMergeCost + count * per * d->d / (1 << 17) : 0;
         int64_t worst = len[0].first, at = count - 1;
+        if (count > 2 * kCUs) {  // the longest of each round of kCUs
+            int64_t sum = 0, c = 0, first = 0;
+            for (int t = 0; t < ntiles; t++)
+                for (c += len[t].second; first < c; first += kCUs) sum += len[t].first;
+            return 16 * sum + merge;
+        }
         // past a workgroup a unit, the k-th longest of the rest joins the k-th shortest of the first
         int i = 0, j = ntiles - 1;
         int64_t ci = len[0].second, cj = count - len[ntiles - 1].second;
@@ -536,23 +555,23 @@ static size_t fwd_split(const dm_attention_desc *d, char *base, FwdSplit *sp) {
             worst = std::max<int64_t>(worst, len[i].first + len[j].first);
             at--;
         }
-        return worst;
+        return 16 * worst + merge;
     };
-    int best = most;
-    int64_t least = ends(most) * 7 / 8 - kMergeCost;  // an eighth to gain, or whole
+    int best = 0;
+    int64_t least = ends(most) * (two ? 12 : 14) / 16;  // an eighth to gain, or whole
     for (int k = 2; k <= 16; k++) {
         const int s = (most + k - 1) / k;
         if (s < kMinTiles) break;
         const int64_t e = ends(s);
-        if (e < least) least = e, best = s;
+        if (e >= 0 && e < least) least = e, best = s;
     }
+    if (best == 0) return 0;
     int c = 0;
     for (int t = 0; t < ntiles; t++) {
         sp->first[t] = (uint16_t)c;
         c += (n[t] + best - 1) / best;
     }
     sp->first[ntiles] = (uint16_t)c;
-    if (c == ntiles) return 0;
     sp->nseg = c;
     const size_t on = align_up((size_t)(c * rows * per * d->d) * 4);
     sp->o = (float *)base;

@@ -186,3 +186,25 @@ def test_loss_workspace_bounds(dtype, n, row_chunk, v, d):
     copies = {_lib.DM_BF16: n * d, _lib.DM_F16: 2 * n * d + v * d, _lib.DM_F32: 0}[dtype] * 4
     assert frozen <= (64 << 20) + copies + 2 * block * chunk * 4 + 64 * max(n, 1) + v // 8 + 16 * 256
     assert both <= frozen + (0 if dtype == _lib.DM_F32 else v * d * 4 + 256)
+
+
+def test_forward_split_is_bounded():
+    """The forward is cut along the keys into 1024 workgroups at most (their partial outputs 128 MB and
+    their references), and a packed call of more than two sequences not at all."""
+    rng = np.random.default_rng(5)
+    split = 0
+    for _ in range(3000):
+        d, hq = int(rng.choice([64, 128, 256])), int(rng.choice([1, 2, 4, 8, 11, 16, 64]))
+        tq, tk = (int(np.exp(rng.uniform(2, 11.5))) for _ in range(2))
+        x = _lib.AttentionDesc(b=1, tq=tq, tk=tk if rng.random() < 0.4 else tq, hq=hq, hkv=1, d=d, dtype=_lib.DM_BF16,
+                               mask_kind=_lib.DM_MASK_NONE)
+        x.options.causal = int(rng.random() < 0.6)
+        if rng.random() < 0.3:
+            x.mask_kind, x.nseq = _lib.DM_MASK_PACKED, int(rng.integers(1, 4))
+        nbytes = _lib.lib().dm_attention_fwd_workspace(ctypes.byref(x))
+        split += nbytes > 0
+        queries = 128 if d == 256 else 256
+        assert nbytes <= 1024 * queries * (4 * d + 8) + 512
+        if x.mask_kind == _lib.DM_MASK_PACKED and x.nseq > 2 or x.tk <= 384:
+            assert nbytes == 0
+    assert split > 300

@@ -28,6 +28,8 @@ CASES = [
     ("padding_1700_b3", 3, 1700, 1700, 1, 1, "padding", False, None, None),
     ("packed_3200", 1, None, None, 2, 1, ("packed", [3000, 200], [3000, 200], 30), True, None,
      None),
+    ("packed_1900_1300", 1, None, None, 2, 1, ("packed", [1900, 1300], [1900, 1300], 0), True, None, None),
+    ("packed_200_2300_window", 1, None, None, 2, 1, ("packed", [200, 2300], [300, 2500], 0), True, (1500, U), None),
 ]
 
 
@@ -56,3 +58,21 @@ def test_split_matches_oracle(case, dtype, d):
         print(f"  o {ro:.2e} lse {rl:.2e}")
         assert ro <= 2 * bounds[0] and rl <= 2 * bounds[1] * max(1.0, np.sqrt(k.shape[1] / 64))
         assert np.all(host(go)[el == -np.inf] == 0.0)
+
+
+def test_more_than_two_workgroups_a_unit():
+    """759 workgroups, taken in rounds: the results of the whole call, each within its bound of the exact
+    ones."""
+    d, hq, tq, tk = 64, 11, 1800, 9000
+    q, k, v = (torch.randn(1, t, h, d, device="cuda", dtype=torch.bfloat16, generator=torch.Generator("cuda").manual_seed(t + h))
+               for t, h in ((tq, hq), (tk, 1), (tk, 1)))
+    opts = dm.AttentionOptions(causal=True)
+    desc = ops._attention_desc("attention", q, k, v, dm.AttentionMask.none(), opts, [])
+    lib = _lib.lib()
+    assert lib.dm_attention_fwd_workspace(ctypes.byref(desc)) > 512 * 256 * (4 * d + 8)
+    o, lse = dm.attention_with_lse(q, k, v, None, opts)
+    o1, lse1 = torch.empty_like(o), torch.empty_like(lse)
+    assert lib.dm_attention_fwd(ctypes.byref(desc), q.data_ptr(), k.data_ptr(), v.data_ptr(), o1.data_ptr(),
+                                lse1.data_ptr(), None, 0, torch.cuda.current_stream().cuda_stream) == 0
+    assert errors(host(o), host(o1))[1] <= 4 * BF16.masks[0]
+    assert errors(host(lse), host(lse1))[1] <= 4 * BF16.masks[1] * np.sqrt(tk / 64)

@@ -954,8 +954,8 @@ __global__ __launch_bounds__(256) void gdr_bwd_mats(GdrArgs a, GdrWs w) {
                 const int i = (wave >> 1) * 32 + ti * 16 + 4 * (lane >> 4) + r;
                 const int j = (wave & 1) * 32 + tj * 16 + (lane & 15);
                 const float d = i >= j ? acc[ti][tj][r] : 0.f;
-                DP[i * kChunk + j] = d * expf(i >= j ? (float)(G[i] - G[j]) : 0.f);
                 acc[ti][tj][r] = d * Pg[i * kChunk + j];
+                DP[i * kChunk + j] = d * expf(i >= j ? (float)(G[i] - G[j]) : 0.f);  // (where Pg was)
             }
     row_sums(acc, red[0]);
     col_sums(acc, red[1]);
@@ -988,8 +988,8 @@ __global__ __launch_bounds__(256) void gdr_bwd_mats(GdrArgs a, GdrWs w) {
                 const int i = (wave >> 1) * 32 + ti * 16 + 4 * (lane >> 4) + r;
                 const int j = (wave & 1) * 32 + tj * 16 + (lane & 15);
                 const float d = i > j ? -acc[ti][tj][r] : 0.f;
-                DA[i * kChunk + j] = d * expf(i > j ? (float)(G[i] - G[j]) : 0.f);
                 acc[ti][tj][r] = d * Ag[i * kChunk + j];
+                DA[i * kChunk + j] = d * expf(i > j ? (float)(G[i] - G[j]) : 0.f);  // (where Ag was)
             }
     row_sums(acc, red[2]);
     col_sums(acc, red[3]);
@@ -1210,8 +1210,11 @@ size_t gdr_ws_layout(const dm_gdr_desc *d, bool backward, char *base, GdrWs *w) 
     x.W = rows(C, KP);
     x.KT = rows(KP, C);
     x.UT = rows(VP, C);
-    x.ScT = rows(VP, KP);
-    x.VnT = rows(VP, C);
+    // What a launch writes goes where an earlier one's is done with. The forward alone: the states over
+    // the rows that prep read (kn and vp follow each other). The state pass: V' over U, each lane reading
+    // its values of a chunk before it writes them.
+    x.ScT = !backward && VP * KP <= C * (KP + VP) ? x.kn : rows(VP, KP);
+    x.VnT = x.UT;
     if (backward) {
         x.inv = rows(2, C);
         x.dop = rows(C, VP);
@@ -1220,15 +1223,18 @@ size_t gdr_ws_layout(const dm_gdr_desc *d, bool backward, char *base, GdrWs *w) 
         x.WT = rows(KP, C);
         x.dvlT = rows(VP, C);
         x.F = rows(VP, KP);
-        x.dSnT = rows(VP, KP);
-        x.dVnT = rows(VP, C);
-        x.DPd = rows(C, C);
-        x.dae = rows(C, C);
-        x.gq = rows(C, KP);
-        x.gk = rows(C, KP);
-        x.dw = rows(C, KP);
         x.dgv = rows(C, 1);
         x.part = rows(x.npart, 1);
+        // the reverse state pass as the forward's, and lane by lane too the matrices' gradients; W and
+        // (lam K)^T serve the state pass alone, W^T the reverse one (2048 tokens of 8 heads of 128: 190 ->
+        // 123 MB)
+        x.dVnT = x.dvlT;
+        x.dSnT = x.F;
+        x.DPd = x.P;
+        x.dae = x.Am;
+        x.gq = x.W;
+        x.gk = x.KT;
+        x.dw = x.WT;
     }
     if (w) *w = x;
     return off;

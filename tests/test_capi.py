@@ -208,3 +208,19 @@ def test_forward_split_is_bounded():
         if x.mask_kind == _lib.DM_MASK_PACKED and x.nseq > 2 or x.tk <= 384:
             assert nbytes == 0
     assert split > 300
+
+
+@pytest.mark.parametrize("dk,dv", [(16, 16), (64, 64), (96, 64), (128, 128), (256, 256), (136, 72)])
+def test_f32_chunk_workspace(dk, dv):
+    """The f32 chunked rule holds, per chunk of 64 tokens and head, rows padded to multiples of 64 columns:
+    the forward 4 rows of Dk and 2 of Dv, P and, past 128 x 128, the state; the backward 5 and 4, P, A, T
+    and two states, and the gates' sums."""
+    kp, vp = -(-dk // 64) * 64, -(-dv // 64) * 64
+    for b, t, h in ((1, 2048, 8), (3, 130, 2)):
+        x = _lib.GdrDesc(b=b, t=t, h=h, dk=dk, dv=dv, dtype=_lib.DM_F32, g_dtype=_lib.DM_F32, beta_dtype=_lib.DM_F32)
+        chunks = b * -(-t // 64) * h
+        rows = lambda k, v: 64 * (k * kp + v * vp)  # noqa: E731
+        fwd = rows(4, 2) + 64 * 64 + 64 * 2 + (vp * kp if vp * kp > 64 * (kp + vp) else 0)
+        bwd = rows(5, 4) + 3 * 64 * 64 + 2 * vp * kp + 64 * 5 + 64 * (6 * kp // 64 + vp // 64 + 1)
+        for size, want in ((_lib.lib().dm_gdr_chunk_fwd_workspace, fwd), (_lib.lib().dm_gdr_chunk_bwd_workspace, bwd)):
+            assert size(ctypes.byref(x)) <= chunks * want * 4 + 24 * 256

@@ -113,6 +113,7 @@ def bench_attention(torch, dm, ops, lib, data, steps, warmup, cu=None, opts=None
     opts = opts or dm.AttentionOptions(causal=True)
     keep = []
     desc = ops._attention_desc("attention", q, k, v, mask, opts, keep)
+    ops._confirm(keep)
     o = torch.empty_like(q)
     lse = torch.empty(q.shape[:3], dtype=torch.float32, device=q.device)
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
@@ -230,6 +231,7 @@ def ref_shapes(torch, dm, ops, lib, syn, dev, args):
         args_t = [c[x] for x in ("q", "k", "v", "g", "beta")]
         desc, _, _ = ops._gdr_desc("chunk_gated_delta_rule", *args_t, c["cu_seqlens"], False,
                                    None, False, keep)
+        ops._confirm(keep)
         outg, fin = torch.empty_like(c["v"]), torch.empty_like(c["h0"])
         nb = lib.dm_gdr_chunk_fwd_workspace(ctypes.byref(desc))
         ws = torch.empty(max(nb, 1), dtype=torch.uint8, device=dev)
@@ -490,6 +492,7 @@ def main():
         args_t = [c[x] for x in ("q", "k", "v", "g", "beta")]
         desc, nseq, (b, t, h, dk, dv) = ops._gdr_desc("chunk_gated_delta_rule", *args_t,
                                                       c["cu_seqlens"], False, None, False, keep)
+        ops._confirm(keep)
         out = torch.empty_like(c["v"])
         fin = torch.empty_like(c["h0"])
         nb = lib.dm_gdr_chunk_fwd_workspace(ctypes.byref(desc))

@@ -44,7 +44,11 @@ def _stream():
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
-def _check(op, rc):
+def _launch(op, keep, fn, *args):
+    """The library call ``fn(*args)`` of a descriptor whose tensors are in ``keep``, after the checks left
+    there (``_confirm``): the one way to the kernels, so that no call goes by them."""
+    _confirm(keep)
+    rc = fn(*args)
     if rc == _lib.DM_OK:
         return
     msg = _lib.last_error()
@@ -143,7 +147,7 @@ def _cu_seqlens(op, t, device, tokens, exact=True, what="cu_seqlens", keep=None)
     at ``tokens`` (``exact``) or, for attention's packed mask, at most there (positions past the
     last offset belong to no sequence, crates/dash-contract/src/attention.rs:49-54). Offsets the
     kernels would index rows with are never passed on unchecked: those already an int32 array on
-    the GPU leave their check in ``keep`` for ``_confirm``. Returns the int32 device array."""
+    the GPU leave their check in ``keep`` for ``_launch``. Returns the int32 device array."""
     def check(cu):
         ok = (len(cu) >= 1 and cu[0] == 0 and all(a <= b for a, b in zip(cu, cu[1:]))
               and (cu[-1] == tokens if exact else cu[-1] <= tokens))
@@ -238,9 +242,8 @@ def attention_with_lse(query, key, value, mask: Optional[AttentionMask] = None,
     lse = torch.empty(q.shape[:3], dtype=torch.float32, device=q.device)
     nbytes = _lib.lib().dm_attention_fwd_workspace(ctypes.byref(desc))
     ws = _workspace(nbytes, q.device)
-    _confirm(keep)
-    _check(op, _lib.lib().dm_attention_fwd(ctypes.byref(desc), _ptr(q), _ptr(k), _ptr(v),
-                                           _ptr(out), _ptr(lse), _ptr(ws), nbytes, _stream()))
+    _launch(op, keep, _lib.lib().dm_attention_fwd, ctypes.byref(desc), _ptr(q), _ptr(k), _ptr(v),
+            _ptr(out), _ptr(lse), _ptr(ws), nbytes, _stream())
     return out, lse
 
 
@@ -272,10 +275,8 @@ def attention_backward(query, key, value, output, lse, grad_output, mask=None, o
     dq, dk, dv = (torch.empty(x.shape, dtype=x.dtype, device=x.device) for x in (q, k, v))
     nbytes = _lib.lib().dm_attention_bwd_workspace(ctypes.byref(desc))
     ws = _workspace(nbytes, q.device)
-    _confirm(keep)
-    _check(op, _lib.lib().dm_attention_bwd(ctypes.byref(desc), _ptr(q), _ptr(k), _ptr(v),
-                                           _ptr(o), _ptr(ls), _ptr(g), _ptr(dq), _ptr(dk),
-                                           _ptr(dv), _ptr(ws), nbytes, _stream()))
+    _launch(op, keep, _lib.lib().dm_attention_bwd, ctypes.byref(desc), _ptr(q), _ptr(k), _ptr(v),
+            _ptr(o), _ptr(ls), _ptr(g), _ptr(dq), _ptr(dk), _ptr(dv), _ptr(ws), nbytes, _stream())
     return dq, dk, dv
 
 
@@ -305,9 +306,8 @@ def attention_decode(query, key, value, lengths=None, options=None):
     out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
     nbytes = _lib.lib().dm_attention_decode_workspace(ctypes.byref(desc))
     ws = _workspace(nbytes, q.device)
-    _confirm(keep)
-    _check(op, _lib.lib().dm_attention_decode(ctypes.byref(desc), _ptr(q), _ptr(k), _ptr(v),
-                                              _ptr(ln), _ptr(out), _ptr(ws), nbytes, _stream()))
+    _launch(op, keep, _lib.lib().dm_attention_decode, ctypes.byref(desc), _ptr(q), _ptr(k),
+            _ptr(v), _ptr(ln), _ptr(out), _ptr(ws), nbytes, _stream())
     return out
 
 
@@ -397,9 +397,8 @@ def attention_decode_packed(query, key, value, cu_seqlens_k, lengths=None, optio
     _decode_strides(desc, q, k, v, (None, 0, 1))
     nbytes = _lib.lib().dm_attention_decode_workspace(ctypes.byref(desc))
     ws = _workspace(nbytes, q.device)
-    _confirm(keep)
-    _check(op, _lib.lib().dm_attention_decode(ctypes.byref(desc), _ptr(q), _ptr(k), _ptr(v),
-                                              _ptr(ln), _ptr(out), _ptr(ws), nbytes, _stream()))
+    _launch(op, keep, _lib.lib().dm_attention_decode, ctypes.byref(desc), _ptr(q), _ptr(k),
+            _ptr(v), _ptr(ln), _ptr(out), _ptr(ws), nbytes, _stream())
     return out
 
 
@@ -432,10 +431,9 @@ def attention_decode_paged(query, key_pages, value_pages, block_table, lengths=N
     out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
     nbytes = _lib.lib().dm_attention_decode_paged_workspace(ctypes.byref(desc), page_size)
     ws = _workspace(nbytes, q.device)
-    _confirm(keep)
-    _check(op, _lib.lib().dm_attention_decode_paged(
-        ctypes.byref(desc), _ptr(q), _ptr(k), _ptr(v), npages, page_size, _ptr(bt), max_pages,
-        _ptr(ln), _ptr(out), _ptr(ws), nbytes, _stream()))
+    _launch(op, keep, _lib.lib().dm_attention_decode_paged, ctypes.byref(desc), _ptr(q), _ptr(k),
+            _ptr(v), npages, page_size, _ptr(bt), max_pages, _ptr(ln), _ptr(out), _ptr(ws), nbytes,
+            _stream())
     return out
 
 
@@ -520,10 +518,9 @@ def chunk_gated_delta_rule(q, k, v, g, beta, initial_state=None, cu_seqlens=None
         if options.output_final_state else None
     nbytes = _lib.lib().dm_gdr_chunk_fwd_workspace(ctypes.byref(desc))
     ws = _workspace(nbytes, q.device)
-    _confirm(keep)
-    _check(op, _lib.lib().dm_gdr_chunk_fwd(ctypes.byref(desc), _ptr(qc), _ptr(kc), _ptr(vc),
-                                           _ptr(gc), _ptr(bc), _ptr(h0), _ptr(out), _ptr(fin),
-                                           _ptr(ws), nbytes, _stream()))
+    _launch(op, keep, _lib.lib().dm_gdr_chunk_fwd, ctypes.byref(desc), _ptr(qc), _ptr(kc),
+            _ptr(vc), _ptr(gc), _ptr(bc), _ptr(h0), _ptr(out), _ptr(fin), _ptr(ws), nbytes,
+            _stream())
     return out, fin
 
 
@@ -555,11 +552,9 @@ def chunk_gated_delta_rule_backward(q, k, v, g, beta, initial_state, cu_seqlens,
         if initial_state is not None else None
     nbytes = _lib.lib().dm_gdr_chunk_bwd_workspace(ctypes.byref(desc))
     ws = _workspace(nbytes, q.device)
-    _confirm(keep)
-    _check(op, _lib.lib().dm_gdr_chunk_bwd(
-        ctypes.byref(desc), _ptr(qc), _ptr(kc), _ptr(vc), _ptr(gc), _ptr(bc), _ptr(h0),
-        _ptr(do), _ptr(dfin), _ptr(dq), _ptr(dk_), _ptr(dv_), _ptr(dg), _ptr(db), _ptr(dh0),
-        _ptr(ws), nbytes, _stream()))
+    _launch(op, keep, _lib.lib().dm_gdr_chunk_bwd, ctypes.byref(desc), _ptr(qc), _ptr(kc),
+            _ptr(vc), _ptr(gc), _ptr(bc), _ptr(h0), _ptr(do), _ptr(dfin), _ptr(dq), _ptr(dk_),
+            _ptr(dv_), _ptr(dg), _ptr(db), _ptr(dh0), _ptr(ws), nbytes, _stream())
     return dq, dk_, dv_, dg, db, dh0
 
 
@@ -590,10 +585,8 @@ def gated_delta_step(q, k, v, g, beta, state, cu_seqlens=None,
         st_in = state.contiguous()
         st_out = torch.empty_like(st_in)
     out = torch.empty((b, h, dv), dtype=q.dtype, device=q.device)
-    _confirm(keep)
-    _check(op, _lib.lib().dm_gdr_step(ctypes.byref(desc), _ptr(qc), _ptr(kc), _ptr(vc),
-                                      _ptr(gc), _ptr(bc), _ptr(st_in), _ptr(st_out), _ptr(out),
-                                      _stream()))
+    _launch(op, keep, _lib.lib().dm_gdr_step, ctypes.byref(desc), _ptr(qc), _ptr(kc), _ptr(vc),
+            _ptr(gc), _ptr(bc), _ptr(st_in), _ptr(st_out), _ptr(out), _stream())
     return out, st_out
 
 
@@ -634,11 +627,9 @@ def gated_delta_step_backward(q, k, v, g, beta, state, cu_seqlens, d_out, d_stat
     dst_in = torch.empty_like(st_in)
     nbytes = _lib.lib().dm_gdr_step_bwd_workspace(ctypes.byref(desc))
     ws = _workspace(nbytes, q.device)
-    _confirm(keep)
-    _check(op, _lib.lib().dm_gdr_step_bwd(
-        ctypes.byref(desc), _ptr(qc), _ptr(kc), _ptr(vc), _ptr(g), _ptr(beta), _ptr(st_in),
-        _ptr(do), _ptr(dst), _ptr(dq), _ptr(dk_), _ptr(dv_), _ptr(dg), _ptr(db), _ptr(dst_in),
-        _ptr(ws), nbytes, _stream()))
+    _launch(op, keep, _lib.lib().dm_gdr_step_bwd, ctypes.byref(desc), _ptr(qc), _ptr(kc), _ptr(vc),
+            _ptr(g), _ptr(beta), _ptr(st_in), _ptr(do), _ptr(dst), _ptr(dq), _ptr(dk_), _ptr(dv_),
+            _ptr(dg), _ptr(db), _ptr(dst_in), _ptr(ws), nbytes, _stream())
     return dq, dk_, dv_, dg, db, dst_in
 
 
@@ -728,9 +719,8 @@ def causal_conv1d(x, weight, bias=None, initial_state=None, cu_seqlens=None,
     bc = None if bias is None else bias.contiguous()
     h0 = None if initial_state is None else initial_state.contiguous()
     out = torch.empty_like(xc)
-    _confirm(keep)
-    _check(op, _lib.lib().dm_causal_conv1d_fwd(ctypes.byref(desc), _ptr(xc), _ptr(wc), _ptr(bc),
-                                               _ptr(h0), _ptr(out), _ptr(fin), _stream()))
+    _launch(op, keep, _lib.lib().dm_causal_conv1d_fwd, ctypes.byref(desc), _ptr(xc), _ptr(wc),
+            _ptr(bc), _ptr(h0), _ptr(out), _ptr(fin), _stream())
     return out, fin
 
 
@@ -765,11 +755,9 @@ def causal_conv1d_backward(x, weight, bias, initial_state, cu_seqlens, grad_out,
     gb = None if bias is None else torch.empty_like(bc)
     gh = None if initial_state is None else torch.empty_like(h0)
     ws = _workspace(_lib.lib().dm_causal_conv1d_bwd_workspace(ctypes.byref(desc)), x.device)
-    _confirm(keep)
-    _check(op, _lib.lib().dm_causal_conv1d_bwd(
-        ctypes.byref(desc), _ptr(xc), _ptr(wc), _ptr(bc), _ptr(h0), _ptr(gc),
-        _DT[grad_out.dtype], _ptr(gf), _ptr(gx), _ptr(gw), _ptr(gb), _ptr(gh), _ptr(ws),
-        ws.numel(), _stream()))
+    _launch(op, keep, _lib.lib().dm_causal_conv1d_bwd, ctypes.byref(desc), _ptr(xc), _ptr(wc),
+            _ptr(bc), _ptr(h0), _ptr(gc), _DT[grad_out.dtype], _ptr(gf), _ptr(gx), _ptr(gw),
+            _ptr(gb), _ptr(gh), _ptr(ws), ws.numel(), _stream())
     return gx, gw, gb, gh
 
 
@@ -798,9 +786,8 @@ def causal_conv1d_update(x, weight, bias, state,
         st_in = state.contiguous()
         st_out = torch.empty_like(st_in)
     out = torch.empty_like(xc)
-    _check(op, _lib.lib().dm_causal_conv1d_update(ctypes.byref(desc), _ptr(xc), _ptr(wc),
-                                                  _ptr(bc), _ptr(st_in), _ptr(out), _ptr(st_out),
-                                                  _stream()))
+    _launch(op, keep, _lib.lib().dm_causal_conv1d_update, ctypes.byref(desc), _ptr(xc), _ptr(wc),
+            _ptr(bc), _ptr(st_in), _ptr(out), _ptr(st_out), _stream())
     return out, st_out
 
 
@@ -847,10 +834,9 @@ def _logprob(hidden, weight, targets, masked, options, with_grad):
     grad = torch.empty(n, d, dtype=torch.float32, device=h.device) if with_grad else None
     nbytes = _lib.lib().dm_chosen_logprob_workspace(ctypes.byref(desc), int(with_grad))
     ws = _workspace(nbytes, h.device)
-    _check(op, _lib.lib().dm_chosen_logprob(ctypes.byref(desc), _ptr(h), _ptr(w), _ptr(tg),
-                                            ctypes.cast(ids_c, ctypes.c_void_p), len(ids),
-                                            _ptr(lp), _ptr(ent), _ptr(grad), _ptr(ws), nbytes,
-                                            _stream()))
+    _launch(op, (), _lib.lib().dm_chosen_logprob, ctypes.byref(desc), _ptr(h), _ptr(w), _ptr(tg),
+            ctypes.cast(ids_c, ctypes.c_void_p), len(ids), _ptr(lp), _ptr(ent), _ptr(grad),
+            _ptr(ws), nbytes, _stream())
     return lp, ent, grad
 
 
@@ -915,9 +901,9 @@ def linear_cross_entropy(hidden, weight, targets, options=None):
     rows = torch.zeros(len(_LCE_ROWS), n, dtype=torch.float32, device=h.device)
     nbytes = _lib.lib().dm_linear_cross_entropy_workspace(ctypes.byref(desc), 0)
     ws = _workspace(nbytes, h.device)
-    _check(op, _lib.lib().dm_linear_cross_entropy_fwd(
-        ctypes.byref(desc), _ptr(h), _ptr(w), _ptr(tg), ctypes.cast(ids_c, ctypes.c_void_p), nid,
-        _ptr(rows), _ptr(ws), nbytes, _stream()))
+    _launch(op, (), _lib.lib().dm_linear_cross_entropy_fwd, ctypes.byref(desc), _ptr(h), _ptr(w),
+            _ptr(tg), ctypes.cast(ids_c, ctypes.c_void_p), nid, _ptr(rows), _ptr(ws), nbytes,
+            _stream())
     if options.reduction == Reduction.NONE:
         loss = rows[0]
     elif options.reduction == Reduction.SUM:
@@ -945,7 +931,7 @@ def linear_cross_entropy_backward(hidden, weight, targets, rows, upstream, optio
     nbytes = _lib.lib().dm_linear_cross_entropy_workspace(ctypes.byref(desc),
                                                           1 if grad_weight else 2)
     ws = _workspace(nbytes, h.device)
-    _check(op, _lib.lib().dm_linear_cross_entropy_bwd(
-        ctypes.byref(desc), _ptr(h), _ptr(w), _ptr(tg), ctypes.cast(ids_c, ctypes.c_void_p), nid,
-        _ptr(rows.contiguous()), _ptr(up), _ptr(gh), _ptr(gw), _ptr(ws), nbytes, _stream()))
+    _launch(op, (), _lib.lib().dm_linear_cross_entropy_bwd, ctypes.byref(desc), _ptr(h), _ptr(w),
+            _ptr(tg), ctypes.cast(ids_c, ctypes.c_void_p), nid, _ptr(rows.contiguous()), _ptr(up),
+            _ptr(gh), _ptr(gw), _ptr(ws), nbytes, _stream())
     return gh, gw

@@ -76,3 +76,35 @@ def test_more_than_two_workgroups_a_unit():
                                 lse1.data_ptr(), None, 0, torch.cuda.current_stream().cuda_stream) == 0
     assert errors(host(o), host(o1))[1] <= 4 * BF16.masks[0]
     assert errors(host(lse), host(lse1))[1] <= 4 * BF16.masks[1] * np.sqrt(tk / 64)
+
+
+# (name, B, Tq, Tk, Hq, Hkv, mask spec, causal, window, scale): at width 64, calls of work items
+# enough for two workgroups a compute unit (768, or 257 of one length), whole
+PAIRED = [
+    ("causal_768", 96, 70, 200, 8, 4, None, True, None, None),
+    ("window_768", 48, 300, 300, 8, 2, None, True, (100, U), 0.1),
+    ("padding_768", 96, 90, 130, 8, 1, "padding", False, None, None),
+    ("equal_272", 17, 70, 500, 16, 2, None, False, None, None),
+    ("packed_768", 1, None, None, 256, 16, ("packed", [300, 40, 260], [300, 90, 260], 5), True, None, None),
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", PAIRED, ids=[c[0] for c in PAIRED])
+def test_paired_workgroups_match_oracle(case, dtype):
+    print(f"case {case[0]} {dtype}", flush=True)
+    (q, k, v, _), mask, opts, mk = _build(case, dtype, 64, 9900 + 17 * PAIRED.index(case))
+    desc = ops._attention_desc("attention", q, k, v, mask, opts, [])
+    items = -(-q.shape[1] // 256) * q.shape[0] * q.shape[2]
+    assert items >= 768 or (case[0].startswith("equal") and items > 256)
+    assert _lib.lib().dm_attention_fwd_workspace(ctypes.byref(desc)) == 0, "the call is split"
+    _lib.probe_reset()
+    o, lse = dm.attention_with_lse(q, k, v, mask, opts)
+    torch.cuda.synchronize()
+    assert _lib.probe_counts()["attn_fwd_mfma"] == 1
+    eo, el = oracle.attention_fwd(mk(host(q), host(k), host(v)), "f64")
+    bounds = (BF16 if dtype == torch.bfloat16 else F16).masks
+    ro, rl = errors(host(o), eo)[1], errors(host(lse), el)[1]
+    print(f"  o {ro:.2e} lse {rl:.2e}")
+    assert ro <= 2 * bounds[0] and rl <= 2 * bounds[1] * max(1.0, np.sqrt(k.shape[1] / 64))
+    assert np.all(host(o)[el == -np.inf] == 0.0)

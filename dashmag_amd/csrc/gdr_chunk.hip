@@ -1369,7 +1369,7 @@ int dm_gdr_chunk_fwd(const dm_gdr_desc *d, const void *q, const void *k, const v
         FWD(DM_F16)
     }
 #undef FWD
-    probe_add(DM_PROBE_GDR_CHUNK_FWD, 4);
+    probe_add(DM_PROBE_GDR_CHUNK_FWD, !w.plan.closed + (chunks ? 3 : 1));
     DM_LAUNCH_CHECK("chunk_gated_delta_rule: launch");
     return DM_OK;
 }
@@ -1426,7 +1426,7 @@ int dm_gdr_chunk_bwd(const dm_gdr_desc *d, const void *q, const void *k, const v
         BWD(DM_F16)
     }
 #undef BWD
-    probe_add(DM_PROBE_GDR_CHUNK_BWD, 9);
+    probe_add(DM_PROBE_GDR_CHUNK_BWD, !w.plan.closed + (chunks ? 8 : 2));
     DM_LAUNCH_CHECK("chunk_gated_delta_rule_backward: launch");
     return DM_OK;
 }

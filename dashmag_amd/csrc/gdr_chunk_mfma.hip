@@ -1981,8 +1981,9 @@ int launch_gdr_mfma_fwd(const dm_gdr_desc *d, const void *q, const void *k, cons
             gdr_mfma_state2<DM_F16, kStateParts, true><<<(unsigned)state_grid(seqs), 64 * kStateParts + 128, state_lds(gdr_mfma_state2<DM_F16, kStateParts, true>), st>>>(a, w, h0, final_state, out);
         }
     }
-    probe_add(DM_PROBE_GDR_CHUNK_FWD, 4);
-    probe_add(DM_PROBE_GDR_CHUNK_FWD_MFMA, 4);
+    const uint64_t launches = !w.plan.closed + (chunks ? 2 : 1);
+    probe_add(DM_PROBE_GDR_CHUNK_FWD, launches);
+    probe_add(DM_PROBE_GDR_CHUNK_FWD_MFMA, launches);
     DM_LAUNCH_CHECK("chunk_gated_delta_rule: MFMA launch");
     return DM_OK;
 }
@@ -2038,8 +2039,9 @@ int launch_gdr_mfma_bwd(const dm_gdr_desc *d, const void *q, const void *k, cons
     else
         gdr_mfma_bwd_kernels<DM_F16>(a, w, chunks, seqs, h0, d_out, d_final, dq, dk, dv, dg,
                                      dbeta, dh0, st);
-    probe_add(DM_PROBE_GDR_CHUNK_BWD, 6);
-    probe_add(DM_PROBE_GDR_CHUNK_BWD_MFMA, 6);
+    const uint64_t launches = !w.plan.closed + (chunks ? 5 : 2);
+    probe_add(DM_PROBE_GDR_CHUNK_BWD, launches);
+    probe_add(DM_PROBE_GDR_CHUNK_BWD_MFMA, launches);
     DM_LAUNCH_CHECK("chunk_gated_delta_rule_backward: MFMA launch");
     return DM_OK;
 }

@@ -45,7 +45,7 @@ bool gdr_strides_16b(const dm_gdr_desc *d);
 
 // Which tokens each chunk holds and which chunks each sequence: the arrays gdr_plan writes for
 // packed sequences, or, for a batch of sequences of T tokens, in closed form from its `per` chunks a
-// sequence (a launch and its latency less: 6144 tokens forward 143 -> 137 us).
+// sequence (a launch and its latency less: 6144 tokens forward 143 -> 138 us).
 struct GdrPlan {
     int32_t *seq_chunk0, *chunk_tok0, *chunk_len;  // [S + 1], [chunks], [chunks]
     int32_t *seq_order;                            // [S]: the sequences by chunk count, the most first

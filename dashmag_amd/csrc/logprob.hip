@@ -45,15 +45,7 @@ __device__ __forceinline__ bool lp_masked(const uint32_t *bits, int64_t tok) {
     return (bits[tok >> 5] >> (tok & 31)) & 1u;
 }
 
-// Sum and maximum over the workgroup's 4 wavefronts, in a fixed order.
-__device__ __forceinline__ float lp_block_sum(float x, float *sm) {
-    x = wave_sum(x);
-    const int w = threadIdx.x >> 6;
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) sm[w] = x;
-    __syncthreads();
-    return (sm[0] + sm[1]) + (sm[2] + sm[3]);
-}
+// Sums and maximum over the workgroup's 4 wavefronts, in a fixed order.
 // Four sums at once (sm: 16 floats): one pair of barriers.
 __device__ __forceinline__ void lp_block_sum4(float (&x)[4], float *sm) {
 #pragma unroll

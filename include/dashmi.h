@@ -190,7 +190,8 @@ int dm_stream_synchronize(void *stream);
 int dm_describe(char *buf, size_t len);
 
 /* Launch counters, the probes of attention.rs:158-221, chunk.rs:119-163 and recurrent.rs:41-50:
- * how many kernels of each kind this process launched. */
+ * how many kernels of each kind this process launched (an attention forward split along the keys
+ * counts as one with its merge, a log-probability or loss call as one). */
 typedef enum {
     DM_PROBE_ATTN_FWD_MFMA = 0,
     DM_PROBE_ATTN_FWD_GENERIC,

@@ -84,10 +84,10 @@ def test_chunking_does_not_change_the_answer(chunks):
 
 
 @pytest.mark.parametrize("dtype,n,d,chunks", [
-    ("bf16", 20000, 64, dict(vocab_chunk=128, row_chunk=3072)),  # two groups of rows
+    ("bf16", 20000, 64, dict(vocab_chunk=128, row_chunk=3072)),  # four groups of rows
     ("f16", 20000, 64, dict(vocab_chunk=128, row_chunk=3072)),
     ("f32", 20000, 64, dict(vocab_chunk=128, row_chunk=3072)),
-    ("f32", 16385, 24, dict(vocab_chunk=0, row_chunk=1)),  # the second group of one row
+    ("f32", 16385, 24, dict(vocab_chunk=0, row_chunk=1)),  # a row a group
     ("bf16", 70, 8, dict(vocab_chunk=7, row_chunk=33)),  # rows of the logits' gradient of 14 bytes
 ])
 def test_row_groups_and_odd_chunks(dtype, n, d, chunks):

@@ -36,6 +36,10 @@ constexpr int fwd_waves() { return D == 256 ? 4 : 8; }
 // one a compute unit where all are of one length (no causal mask, window or packing): with fewer, two
 // of the longest share a unit and end the call late (2 x 3072 causal of 16 heads, 384 items, 65 us
 // alone and 80 paired, of 24 heads 101 and 102, of 32 heads, 768 items, 120 and 102).
+// Key padding takes 187 registers freely, and a pair there 1.83 times as long as one: paired where the
+// items are an even number of rounds of the compute units, or more than six (2 x 4096 queries of 64 heads 2083 ->
+// 1824 us, seven rounds of 1024 queries 492 -> 466, but 4 x 2048 of 24 heads, three rounds, 403 -> 448),
+// and never where the call is split, which spills (2 x 3000 causal of 8 heads 105 -> 184).
 template <int D, bool PAIR>
 constexpr int fwd_simd_waves() { return D == 64 && PAIR ? 4 : 1; }
 constexpr int64_t kPairItems = 768;
@@ -604,9 +608,12 @@ int launch_attn_fwd_mfma(const MaskInfo &m, const dm_attention_desc *d, float sc
     uint16_t *oo = (uint16_t *)o;
     const AttnStrides sd = attn_strides(d);
     const bool equal = m.right < 0 && m.left < 0 && m.kind != DM_MASK_PACKED;
-    const bool pair = d->d == 64 && (split || nwork >= kPairItems || (equal && nwork > 256));
+    const int64_t rounds = (nwork + 255) / 256;
+    const bool fits = !m.pad || rounds % 2 == 0 || rounds > 6;
+    const bool pair = d->d == 64 && (split || (fits && (nwork >= kPairItems || (equal && nwork > 256))));
 #define FWD1(DT, DD, PAD, SPLIT)                                                                  \
-    if (pair) FWD2(DT, DD, PAD, SPLIT, DD == 64); else FWD2(DT, DD, PAD, SPLIT, DD == 64 && SPLIT)
+    if (pair) FWD2(DT, DD, PAD, SPLIT, DD == 64 && !(PAD && SPLIT));                              \
+    else FWD2(DT, DD, PAD, SPLIT, DD == 64 && !PAD && SPLIT)
 #define FWD2(DT, DD, PAD, SPLIT, PAIR)                                                            \
     attn_fwd_mfma<DT, DD, PAD, SPLIT, PAIR><<<grid, block, 0, st>>>(m, d->b, d->hq, d->hkv, scale, sd, qq, \
                                                               kk, vv, oo, lse, sp)

@@ -16,7 +16,7 @@
 // left is the chain of a workgroup's first loads, its bounds and the sum at its end.)
 //
 // At 256 tokens of 4 heads of 64, causal, forward and backward took 410 us as one wavefront a row
-// (a dot product, a wavefront reduction and an exponential a key, one after another), and take 47.
+// (a dot product, a wavefront reduction and an exponential a key, one after another), and take 48.
 #include <string>
 
 #include "attention_kernels.h"
@@ -418,13 +418,14 @@ __global__ __launch_bounds__(64 * kNW) void attn_dkdv_f32(AttnF32 a, void *dk, v
     __shared__ int range[2];
     float *os = (float *)os4;
 
-    // the query tiles that see any of the 16 keys lie in [range[0], range[1])
+    const bool pad = j >= Tk || (a.m.pad && a.m.pad[b * Tk + jc]);
+    // the query tiles that see any of the 16 keys lie in [range[0], range[1]) (none where all are padded)
     if (threadIdx.x == 0) {
         range[0] = nt;
         range[1] = 0;
     }
     __syncthreads();
-    for (int t = threadIdx.x; t < nt; t += 64 * kNW) {
+    for (int t = __all(pad) ? nt : threadIdx.x; t < nt; t += 64 * kNW) {
         const int2 u = a.tile[b * nt + t];
         if (u.x < kt * kQT + kQT && u.y > kt * kQT) {
             atomicMin(&range[0], t);
@@ -435,7 +436,6 @@ __global__ __launch_bounds__(64 * kNW) void attn_dkdv_f32(AttnF32 a, void *dk, v
     const int64_t ko = b * a.sd.k.b + jc * a.sd.k.t + kh * a.sd.k.h, vo = b * a.sd.v.b + jc * a.sd.v.t + kh * a.sd.v.h;
     row_load<DT, VEC>(kf, a.k, ko, D, g);
     row_load<DT, VEC>(vf, a.v, vo, D, g);
-    const bool pad = j >= Tk || (a.m.pad && a.m.pad[b * Tk + jc]);
     f32x4_t ak[NS], av[NS];
 #pragma unroll
     for (int s = 0; s < NS; s++) ak[s] = av[s] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -482,7 +482,7 @@ __global__ __launch_bounds__(64 * kNW) void attn_dkdv_f32(AttnF32 a, void *dk, v
         const bool all = all_seen(on);
         if constexpr (kEarly) {
             if (!all) {
-                const Hidden hid(on, j < Tk);
+                const Hidden hid(on, !pad);
                 badq |= hid.clear(qc);
                 badg |= hid.clear(gc);
             }
@@ -505,7 +505,7 @@ __global__ __launch_bounds__(64 * kNW) void attn_dkdv_f32(AttnF32 a, void *dk, v
                 x[0] = col_load<DT>(a.q, qo, 16 * s + c, D);
                 y[0] = col_load<DT>(a.d_o, go, 16 * s + c, D);
                 if (!all) {
-                    const Hidden hid(on, j < Tk);
+                    const Hidden hid(on, !pad);
                     badq |= hid.clear(x);
                     badg |= hid.clear(y);
                 }
@@ -523,7 +523,7 @@ __global__ __launch_bounds__(64 * kNW) void attn_dkdv_f32(AttnF32 a, void *dk, v
             bool on[4];
 #pragma unroll
             for (int r = 0; r < 4; r++) on[r] = sees(record(h, i0 + 4 * g + r));
-            if (!Hidden(on, j < Tk).cut) continue;
+            if (!Hidden(on, !pad).cut) continue;
 #pragma unroll 1
             for (int64_t i = i0; i < i0 + kQT; i++) {
                 const RowRec x = record(h, i);
@@ -542,10 +542,11 @@ __global__ __launch_bounds__(64 * kNW) void attn_dkdv_f32(AttnF32 a, void *dk, v
     const int64_t to = ((b * Tk + kt * kQT + r) * a.Hkv + kh) * D;
     auto give = [&](const f32x4_t (&x)[NS], void *out, float f) {
         __syncthreads();
+        // (a padded key sees nothing, and its column may hold 0 * NaN: its terms were not looked at)
 #pragma unroll
         for (int s = 0; s < NS; s++)
             *(float4 *)(os + (wave * kQT + c) * OS + 16 * s + 4 * g) =
-                make_float4(x[s][0], x[s][1], x[s][2], x[s][3]);
+                pad ? make_float4(0.f, 0.f, 0.f, 0.f) : make_float4(x[s][0], x[s][1], x[s][2], x[s][3]);
         __syncthreads();
         if (kt * kQT + r >= Tk) return;
         for (int d = threadIdx.x % kL; d < D; d += kL) {

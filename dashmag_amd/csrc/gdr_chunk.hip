@@ -120,8 +120,8 @@ __global__ __launch_bounds__(1024) void gdr_plan(int64_t nseq, int64_t T, int64_
 // one-lane-per-element dot products that these replace ran at 0.2 TFLOP/s, every multiply waiting
 // on two loads, with each (sequence, head) on one compute unit in the state passes: forward and
 // backward of 2048 tokens in sequences of 700, 1001 and 347, 8 heads of 128, took 48.4 ms (state
-// passes 11.4 and 16.3 ms, gradients 6.2 ms) and take 0.44 ms (state passes 40 and 47 us, prep 58
-// us, the gradients' four launches 131 us). What bounds a call of that size is latency: 33 chunks of 8 heads are
+// passes 11.4 and 16.3 ms, gradients 6.2 ms) and take 0.44 ms (state passes 40 and 46 us, prep 59
+// us, the gradients' four launches 129 us). What bounds a call of that size is latency: 33 chunks of 8 heads are
 // one workgroup per compute unit, each a chain of panels (load, barrier, products).
 // ------------------------------------------------------------------------------------------
 
